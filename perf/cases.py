@@ -63,28 +63,28 @@ def listed():
     return [
         # One layer of a small request through the drop-in operator: the smallest call a
         # runtime makes, once per layer, where the host path and the launch are the cost.
-        _operator(name="operator, one layer, 2k tokens", layers=1, tokens=2048, mask=True, prefix=512),
+        _operator(name="operator_one_layer_tokens", layers=1, tokens=2048, mask=True, prefix=512),
         # A model whose keys rotate a quarter of their dims (GPT-NeoX, Phi style).
-        _operator(name="operator, quarter rotary", rotary=32),
+        _operator(name="operator_quarter_rotary", rotary=32),
         # A model whose value heads are narrower than its key heads.
-        _operator(name="operator, narrow values", heads=8, value_dim=64),
+        _operator(name="operator_narrow_values", heads=8, value_dim=64),
         # A short chat's link (c1) with the reference's default rounding: latency of the
         # whole call, host preparation included.
-        _link(name="link, 2k tokens", tokens=2048, blocks=4, seam=8, shifted=True, mode="disabled"),
+        _link(name="link_2k_tokens", tokens=2048, blocks=4, seam=8, shifted=True, mode="disabled"),
         # The headline: a 32k-token request of 16 blocks (c2).
-        _link(name="link, 32k tokens"),
+        _link(name="link_32k_tokens"),
         # The same length from many small blocks, half of it repair rows (c5).
-        _link(name="link, 512 blocks", blocks=512, seam=32, shifted=True),
+        _link(name="link_512_blocks", blocks=512, seam=32, shifted=True),
         # A batch of requests that share catalogue blocks (c3): the largest link.
-        _link(name="link, batch of 24", requests=24, tokens=4096, blocks=8, catalogue=64, seam=8),
+        _link(name="link_batch_of_24", requests=24, tokens=4096, blocks=8, catalogue=64, seam=8),
         # One layer's repair attention of c1's, c2's and c5's spans ...
-        _repair(name="repair, 2k tokens", tokens=2048, spans=3, rows=8),
-        _repair(name="repair, 32k tokens"),
-        _repair(name="repair, 512 blocks", spans=511, rows=32),
+        _repair(name="repair_2k_tokens", tokens=2048, spans=3, rows=8),
+        _repair(name="repair_32k_tokens"),
+        _repair(name="repair_512_blocks", spans=511, rows=32),
         # ... of a batch of requests like c3's ...
-        _repair(name="repair, batch of 24", requests=24, tokens=8192, spans=7, rows=8, index="int32"),
+        _repair(name="repair_batch_of_24", requests=24, tokens=8192, spans=7, rows=8, index="int32"),
         # ... and of a model with wide heads in fp16.
-        _repair(name="repair, head dim 256", dim=256, tokens=16384, kv="fp16", q_heads=8),
+        _repair(name="repair_head_dim_256", dim=256, tokens=16384, kv="fp16", q_heads=8),
     ]
 
 

@@ -1,6 +1,6 @@
 // LegoLink KV link kernels for MI355X (gfx950) and their C ABI.
 //
-// Two kernels implement the link (gather -> RoPE delta re-rotation -> scatter):
+// Three kernels implement the link (gather -> RoPE delta re-rotation -> scatter):
 //
 //   kv_link_vec_kernel      the production kernel.  The per-layer K/V rows of
 //                           all tokens are flattened into 16-byte chunks; one
@@ -13,10 +13,14 @@
 //                           q and q ^ (D/16) of the same head, so the partner
 //                           half arrives by a DPP row rotation (D = 128) or a
 //                           lane swizzle (other D) instead of a second load.
+//   kv_link_chunk_kernel    the other shapes whose head dims and rotary halves
+//                           are whole 16-byte chunks (any partial rotary, K/V
+//                           head dims that differ, head dims other than powers
+//                           of two, maps of mixed index types): a lane owns one
+//                           K or one V chunk and loads its rotary partner.
 //   kv_link_generic_kernel  one thread per rotary pair / pass-through element /
 //                           V element; every shape the operator accepts
-//                           (partial rotary, K/V head dims that differ,
-//                           bf16/fp16 caches, strided caches).
+//                           (also odd dims, strided caches, unaligned buffers).
 //
 // kv_scatter_kernel writes repaired boundary rows into the pool.
 //
@@ -97,6 +101,7 @@ struct LinkParams {
   long long k_row_bytes;
   long long v_row_bytes;
   long long chunks_per_row;  // vector kernel: 16-byte chunks per K row (== per V row)
+  unsigned key_waves;        // chunk kernel: waves over the K heads (the V chunks' waves follow)
   int num_layers;            // layers in this launch
   int layers_per_wave;
   int layer_groups_per_block;  // vector kernel: waves of a block that share a token
@@ -786,6 +791,156 @@ __global__ void __launch_bounds__(512) kv_link_generic_kernel(const LinkParams p
 }
 
 // ---------------------------------------------------------------------------
+// Chunk link kernel: shapes outside the vector kernel whose rows are whole
+// 16-byte chunks.  Waves [0, key_waves) cover the K heads of all tokens, as
+// many whole heads per wave as fit its 64 lanes, and the waves after them the
+// V chunks, 64 per wave, so key and value rows may differ in width; grid.y =
+// runs of layers_per_wave layers.  A K lane computes its chunk's RoPE delta
+// once for its run of layers.  Its rotary partner chunk (rotary_dim / 2
+// elements away, in the same head) comes by a second load, which hits the L1:
+// it is another lane's own chunk.  That lane is in the same wave, whose loads
+// of a layer all come before its stores, so a token may also be linked onto
+// its own slot.  Chunks that do not rotate load their own address again.
+//
+// Bound by HBM like the vector kernel: it moves 16 bytes per lane and request
+// and each row byte once.  kv_link_generic_kernel, which took these shapes,
+// moves 2 bytes per lane and request and computes a delta per pair and layer.
+// 28 layers x 8,192 tokens, bf16, fp32 table: 4 heads x 128 with rotary 32,
+// 749 -> 187 us (5.0 TB/s); 8 heads of 128 (K) and 64 (V), 850 -> 283 us (5.0
+// TB/s); a 2 GiB device copy on the same box runs at 4.9 TB/s.
+// Two layers per K lane before its stores: four
+// took 0.5 us more on one layer and 2 % more on 28.
+// Requirements (checked on the host): key_head_dim and value_head_dim
+// multiples of 8, rotary_dim a multiple of 16 (neox) or 8 (GPT-J), a table
+// with unit column stride and 16-byte aligned rows, 16-byte aligned buffers,
+// fewer than 2^31 V chunks (and so K heads) in all.
+// ---------------------------------------------------------------------------
+template <bool kBF16, int kCache, bool kEager, bool kNeox>
+__global__ void __launch_bounds__(512) kv_link_chunk_kernel(const LinkParams p) {
+  using Round = Rounding<kBF16, kCache, kEager>;
+  constexpr int kPairs = kNeox ? 8 : 4;
+  const int lane = threadIdx.x & (kWave - 1);
+  // Wave-uniform: the wave's side (K or V) and layers.
+  const unsigned wave_all = blockIdx.x * (blockDim.x / kWave) +
+                            __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const bool is_key = wave_all < p.key_waves;
+  const unsigned wave = is_key ? wave_all : wave_all - p.key_waves;
+  const int l0 = blockIdx.y * p.layers_per_wave;
+  const int l1 = min(l0 + p.layers_per_wave, p.num_layers);
+  if (l0 >= l1) return;
+  // The lane's token, its chunk c of the token's row and (K) chunk q of its
+  // head, from its unit (a head of K, a chunk of V) of all tokens.
+  const unsigned head_chunks = static_cast<unsigned>(p.kdim) / 8;
+  const unsigned wave_units = is_key ? kWave / head_chunks : kWave;
+  const unsigned row_units = is_key ? static_cast<unsigned>(p.num_heads) : static_cast<unsigned>(p.v_row_bytes / 16);
+  const unsigned lane_unit = is_key ? lane / head_chunks : lane;
+  const unsigned q = lane - lane_unit * head_chunks;  // K only
+  const unsigned unit = wave * wave_units + lane_unit;
+  const unsigned token = unit / row_units;
+  const unsigned row_unit = unit - token * row_units;
+  const bool in_range = lane_unit < wave_units && token < p.num_tokens;
+  const unsigned c = !in_range ? 0 : is_key ? row_unit * head_chunks + q : row_unit;
+  const long long t = in_range ? token : 0;
+
+  // The token's maps and mask byte: independent loads (without a mask, a byte
+  // of the source map is read and ignored).
+  const long long src = load_index(p.src, p.idx64 & 1, t);
+  const long long dst = load_index(p.dst, p.idx64 & 2, t);
+  const long long lp = load_index(p.lpos, p.idx64 & 4, t);
+  const long long gp = load_index(p.gpos, p.idx64 & 8, t);
+  const unsigned char mask_byte =
+      (p.mask != nullptr ? p.mask : static_cast<const unsigned char *>(p.src))[t];
+  const bool remap = t >= p.prefix;
+  const bool positions_ok = lp >= 0 && lp < p.cs_rows && gp >= 0 && gp < p.cs_rows;
+  const bool masked = p.mask != nullptr && mask_byte != 0;
+  const bool ok = in_range && !masked && src >= 0 && src < p.src_num_slots && dst >= 0 &&
+                  dst < p.num_slots && (!remap || positions_ok);
+  // An unmasked token skipped for an out-of-range index is counted once, by
+  // its first K chunk's lane in the first run of layers.
+  if (p.skipped != nullptr && is_key && in_range && !ok && !masked && c == 0 && l0 == 0)
+    atomicAdd(p.skipped, 1ull);
+  // Row loads are unconditional: a token without a valid source reads row 0
+  // (the host launches only when the source pool has rows) and stores nothing.
+  const long long src_row = (src >= 0 && src < p.src_num_slots) ? src : 0;
+
+  constexpr int kUnroll = 2;   // layers of a K lane's loads (two per layer) before its stores
+  constexpr int kUnrollV = 4;
+  if (!is_key) {
+    const long long from = src_row * p.v_row_bytes + static_cast<long long>(c) * 16;
+    const long long to = dst * p.v_row_bytes + static_cast<long long>(c) * 16;
+    for (int l = l0; l < l1; l += kUnrollV) {
+      u32x4 in[kUnrollV];
+#pragma unroll
+      for (int u = 0; u < kUnrollV; ++u) in[u] = load_row<false>(p.sv_layers[min(l + u, l1 - 1)] + from);
+#pragma unroll
+      for (int u = 0; u < kUnrollV; ++u)
+        if (ok && l + u < l1) store_row_chunk(p.v_layers[l + u] + to, in[u]);
+    }
+    return;
+  }
+
+  const bool rotates = in_range && q < static_cast<unsigned>(p.rotary_dim / 8) && remap && positions_ok;
+  const int half = p.rotary_dim / 2;
+  const unsigned half_chunks = static_cast<unsigned>(p.rotary_dim / 16);
+  const bool second_half = kNeox && q >= half_chunks;
+  int partner = 0;  // bytes from the lane's chunk to its rotary partner
+  if (kNeox && rotates) partner = second_half ? -static_cast<int>(half_chunks) * 16 : static_cast<int>(half_chunks) * 16;
+  const long long from = src_row * p.k_row_bytes + static_cast<long long>(c) * 16;
+  const long long to = dst * p.k_row_bytes + static_cast<long long>(c) * 16;
+
+  // The first layers' rows are requested before the table's entries, so both
+  // are in flight together.
+  u32x4 in[kUnroll], other[kUnroll];
+  auto load_rows = [&](int l) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const char *row = p.sk_layers[min(l + u, l1 - 1)] + from;
+      in[u] = load_row<false>(row);
+      if constexpr (kNeox) other[u] = load_row<false>(row + partner);
+    }
+  };
+  load_rows(l0);
+  float dc[kPairs], dsn[kPairs];  // delta cosine and (neox: signed) sine of the lane's pairs
+#pragma unroll
+  for (int e = 0; e < kPairs; ++e) {
+    dc[e] = 1.0f;
+    dsn[e] = 0.0f;
+  }
+  if (rotates) {  // then the table has rows
+    const int pb = kNeox ? static_cast<int>(second_half ? q - half_chunks : q) * 8 : static_cast<int>(q) * 4;
+    const long long lrow = lp * p.cs_stride_row + pb;
+    const long long grow = gp * p.cs_stride_row + pb;
+    float lc[kPairs], ls[kPairs], gc[kPairs], gs[kPairs];
+    load_table<kCache, kPairs>(p.cs, lrow, lc);
+    load_table<kCache, kPairs>(p.cs, lrow + half, ls);
+    load_table<kCache, kPairs>(p.cs, grow, gc);
+    load_table<kCache, kPairs>(p.cs, grow + half, gs);
+#pragma unroll
+    for (int e = 0; e < kPairs; ++e) {
+      float ds;
+      delta_pair<Round::kDelta, Round::kCast>(lc[e], ls[e], gc[e], gs[e], dc[e], ds);
+      dsn[e] = kNeox && !second_half ? -ds : ds;
+    }
+  }
+  // Scalars from here on: paired into two-element vectors, fp16 GPT-J deltas
+  // end in a negation that this compiler cannot select without packed fp32.
+#pragma unroll
+  for (int e = 0; e < kPairs; ++e) asm("" : "+v"(dc[e]), "+v"(dsn[e]));
+  for (int l = l0; l < l1; l += kUnroll) {
+    if (l != l0) load_rows(l);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      u32x4 out = in[u];
+      if (rotates) {
+        if constexpr (kNeox) out = rotate_neox<kBF16, Round::kProd>(in[u], other[u], dc, dsn);
+        else out = rotate_gptj<kBF16, Round::kProd>(in[u], dc, dsn);
+      }
+      if (ok && l + u < l1) store_row_chunk(p.k_layers[l + u] + to, out);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Repaired-row scatter: grid.y = layer; threads stride over the layer's
 // (row, chunk) items, K rows first, then V rows.
 // ---------------------------------------------------------------------------
@@ -1115,16 +1270,9 @@ int validate_link(const ll_kv_link_args *a) {
   return LL_OK;
 }
 
-bool vector_kernel_fits(const ll_kv_link_args *a) {
-  const int64_t d = a->key_head_dim;
-  // One index type for all four token maps.
-  if (a->destination_slots_dtype != a->source_slots_dtype ||
-      a->local_positions_dtype != a->source_slots_dtype ||
-      a->global_positions_dtype != a->source_slots_dtype)
-    return false;
-  if (!(d == 32 || d == 64 || d == 128 || d == 256)) return false;
-  if (a->value_head_dim != d) return false;
-  if (a->rotary_dim != d && !(a->rotary_dim * 2 == d && d >= 32)) return false;
+// 16-byte row chunks and table reads: unit-stride table rows and every buffer
+// 16-byte aligned.
+bool chunk_access_fits(const ll_kv_link_args *a) {
   if (a->cos_sin_stride_col != 1 || !aligned16(a->cos_sin_cache)) return false;
   // Rows 16-byte aligned: 4 fp32 or 8 16-bit entries per 16 bytes.
   if ((a->cos_sin_stride_row % (a->cos_sin_dtype == LL_DTYPE_FLOAT32 ? 4 : 8)) != 0) return false;
@@ -1136,12 +1284,41 @@ bool vector_kernel_fits(const ll_kv_link_args *a) {
   return true;
 }
 
+bool vector_kernel_fits(const ll_kv_link_args *a) {
+  const int64_t d = a->key_head_dim;
+  // One index type for all four token maps.
+  if (a->destination_slots_dtype != a->source_slots_dtype ||
+      a->local_positions_dtype != a->source_slots_dtype ||
+      a->global_positions_dtype != a->source_slots_dtype)
+    return false;
+  if (!(d == 32 || d == 64 || d == 128 || d == 256)) return false;
+  if (a->value_head_dim != d) return false;
+  if (a->rotary_dim != d && !(a->rotary_dim * 2 == d && d >= 32)) return false;
+  return chunk_access_fits(a);
+}
+
+// The chunk kernel takes what the vector kernel does not, where a head's dims
+// and (neox) each rotary half, or (GPT-J) the rotary dims, are whole 16-byte
+// chunks; a GPT-J lane then reads four table entries, 16 bytes of fp32 or 8 of
+// a 16-bit table.  No size bounds it: from one layer x 1 token to one layer x
+// 256 tokens the two general kernels take the same time (3.1-4.0 us, within
+// 0.4 us of each other), at one layer x 2,048 it takes 4.3-5.4 us against
+// 5.9-7.7, and at 28 layers x 256 and more it is 1.7 to 8.6 times as fast.
+bool chunk_kernel_fits(const ll_kv_link_args *a) {
+  return a->key_head_dim % 8 == 0 && a->value_head_dim % 8 == 0 &&
+         a->rotary_dim % (a->is_neox_style ? 16 : 8) == 0 &&
+         a->num_heads <= (1 << 20) && a->num_tokens <= 0x7fffffff &&
+         a->num_tokens * a->num_heads * (a->value_head_dim / 8) <= 0x7fffffff && chunk_access_fits(a);
+}
+
 struct LinkPlan {
   int kernel;  // LL_KERNEL_VECTOR / LL_KERNEL_GENERIC
+  bool chunked;  // LL_KERNEL_GENERIC by the chunk kernel
   int block_threads;
   long long grid_x;
   int layers_per_wave;  // vector kernel
   int layer_groups_per_block;  // vector kernel
+  long long key_waves;  // chunk kernel
   int launches;
   bool staged;  // vector kernel: workgroup-staged deltas
   bool layer_major;  // delta table + layer-major kernel
@@ -1170,6 +1347,14 @@ bool table_fits(const ll_kv_link_args *a) {
 constexpr long long kTargetWaves = 16384;  // 64 waves per CU on 256 CUs
 constexpr int kDefaultLayersPerWave = 4;
 
+int default_layers_per_wave(long long waves_x, int layers) {
+  if (waves_x * ((layers + kDefaultLayersPerWave - 1) / kDefaultLayersPerWave) >= kTargetWaves)
+    return kDefaultLayersPerWave;
+  long long groups = (kTargetWaves + waves_x - 1) / waves_x;
+  if (groups > layers) groups = layers;
+  return static_cast<int>((layers + groups - 1) / groups);
+}
+
 int plan_link(const ll_kv_link_args *a, LinkPlan *plan) {
   const bool fits = vector_kernel_fits(a);
   if (a->kernel == LL_KERNEL_VECTOR && !fits)
@@ -1184,6 +1369,22 @@ int plan_link(const ll_kv_link_args *a, LinkPlan *plan) {
   const int layers_first = static_cast<int>(
       a->num_layers < kMaxLayersPerLaunch ? a->num_layers : kMaxLayersPerLaunch);
   plan->launches = static_cast<int>((a->num_layers + kMaxLayersPerLaunch - 1) / kMaxLayersPerLaunch);
+  // An explicit LL_KERNEL_GENERIC asks for the one-thread-per-pair kernel.
+  plan->chunked = plan->kernel == LL_KERNEL_GENERIC && a->kernel == LL_KERNEL_AUTO && chunk_kernel_fits(a);
+  if (plan->chunked) {
+    const int64_t wave_heads = kWave / (a->key_head_dim / 8);
+    plan->key_waves = (a->num_tokens * a->num_heads + wave_heads - 1) / wave_heads;
+    const long long waves_x =
+        plan->key_waves + (a->num_tokens * (a->num_heads * a->value_head_dim / 8) + kWave - 1) / kWave;
+    plan->grid_x = (waves_x + waves_per_block - 1) / waves_per_block;
+    plan->layers_per_wave = a->layers_per_wave ? static_cast<int>(std::min<int64_t>(a->layers_per_wave, layers_first))
+                                               : default_layers_per_wave(waves_x, layers_first);
+    plan->layer_groups_per_block = 1;
+    plan->staged = false;
+    plan->layer_major = false;
+    if (plan->grid_x <= 0x7fffffffLL) return LL_OK;
+    plan->chunked = false;  // the generic kernel's blocks stride over any number of tokens
+  }
   if (plan->kernel == LL_KERNEL_VECTOR) {
     const long long chunks = a->num_heads * a->key_head_dim / 8;
     const long long waves_x = (a->num_tokens * chunks + kWave - 1) / kWave;
@@ -1193,16 +1394,7 @@ int plan_link(const ll_kv_link_args *a, LinkPlan *plan) {
     const int chunk_waves_per_block = waves_per_block / groups_per_block;
     plan->grid_x = (waves_x + chunk_waves_per_block - 1) / chunk_waves_per_block;
     int lpw = static_cast<int>(a->layers_per_wave);
-    if (lpw == 0) {
-      if (waves_x * ((layers_first + kDefaultLayersPerWave - 1) / kDefaultLayersPerWave) >=
-          kTargetWaves) {
-        lpw = kDefaultLayersPerWave;
-      } else {
-        long long groups = (kTargetWaves + waves_x - 1) / waves_x;
-        if (groups > layers_first) groups = layers_first;
-        lpw = static_cast<int>((layers_first + groups - 1) / groups);
-      }
-    }
+    if (lpw == 0) lpw = default_layers_per_wave(waves_x, layers_first);
     if (lpw > layers_first) lpw = layers_first;
     plan->layers_per_wave = lpw;
     plan->staged = false;
@@ -1381,6 +1573,26 @@ void launch_layer_major(bool bf16, dim3 grid, hipStream_t s, const LinkParams &p
   }
 }
 
+template <bool kBF16, int kCache>
+void launch_chunk_cache(dim3 grid, dim3 block, hipStream_t s, const LinkParams &p) {
+  if (p.eager) {
+    if (p.neox) kv_link_chunk_kernel<kBF16, kCache, true, true><<<grid, block, 0, s>>>(p);
+    else kv_link_chunk_kernel<kBF16, kCache, true, false><<<grid, block, 0, s>>>(p);
+  } else {
+    if (p.neox) kv_link_chunk_kernel<kBF16, kCache, false, true><<<grid, block, 0, s>>>(p);
+    else kv_link_chunk_kernel<kBF16, kCache, false, false><<<grid, block, 0, s>>>(p);
+  }
+}
+
+template <bool kBF16>
+void launch_chunk(int cache_dtype, dim3 grid, dim3 block, hipStream_t s, const LinkParams &p) {
+  switch (cache_dtype) {
+    case LL_DTYPE_FLOAT32: launch_chunk_cache<kBF16, 3>(grid, block, s, p); break;
+    case LL_DTYPE_BFLOAT16: launch_chunk_cache<kBF16, 2>(grid, block, s, p); break;
+    default: launch_chunk_cache<kBF16, 1>(grid, block, s, p); break;
+  }
+}
+
 template <int kKey, bool kEager>
 void launch_generic_cache(int cache_dtype, dim3 grid, dim3 block, hipStream_t s,
                           const LinkParams &p) {
@@ -1471,7 +1683,7 @@ int ll_kv_link_describe(const ll_kv_link_args *args, ll_launch_info *info) {
   info->launches = plan.launches;
   info->grid_x = plan.grid_x;
   const int layer_groups = (layers_first + plan.layers_per_wave - 1) / plan.layers_per_wave;
-  info->grid_y = plan.kernel == LL_KERNEL_VECTOR
+  info->grid_y = plan.kernel == LL_KERNEL_VECTOR || plan.chunked
                      ? (layer_groups + plan.layer_groups_per_block - 1) / plan.layer_groups_per_block
                      : layers_first;
   info->block_threads = plan.block_threads;
@@ -1567,6 +1779,14 @@ int ll_kv_link(const ll_kv_link_args *a, ll_stream_t stream) {
       const int cache = static_cast<int>(a->cos_sin_dtype);
       if (bf16) launch_vec<true>(cache, p.kdim, grid, block, s, p, p.neox != 0);
       else launch_vec<false>(cache, p.kdim, grid, block, s, p, p.neox != 0);
+    } else if (plan.chunked) {
+      p.layers_per_wave = plan.layers_per_wave;
+      p.layer_groups_per_block = 1;
+      p.key_waves = static_cast<unsigned>(plan.key_waves);
+      const dim3 grid(static_cast<unsigned>(plan.grid_x),
+                      static_cast<unsigned>((n + plan.layers_per_wave - 1) / plan.layers_per_wave));
+      if (bf16) launch_chunk<true>(static_cast<int>(a->cos_sin_dtype), grid, block, s, p);
+      else launch_chunk<false>(static_cast<int>(a->cos_sin_dtype), grid, block, s, p);
     } else {
       p.layers_per_wave = 1;
       p.layer_groups_per_block = 1;

@@ -149,11 +149,6 @@ struct F16 {
   }
 };
 
-__device__ inline long long slot_at(const AttnParams &p, long long i) {
-  return p.slots64 ? static_cast<const long long *>(p.slots)[i]
-                   : static_cast<long long>(static_cast<const int *>(p.slots)[i]);
-}
-
 // Partial result of item `partial`, query head h: the 16 queries' outputs
 // over the item's keys, normalised by their own sums (O / l) and rounded to
 // the KV dtype, [16][D] 16-bit values, then (m, l) [16][2] in fp32: 8 D + 32
@@ -340,9 +335,29 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   __shared__ unsigned long long tile_valid[kRangeTiles];
 
   constexpr int kPairs = max_pairs(D);
-  const int *it = p.items + static_cast<long long>(blockIdx.x) * kItemInts;
-  const int kv_off = it[0], kv_begin = it[1], kv_end = it[2], n_tiles = it[3];
-  const int pair_first = it[4], pair_count = it[5];
+  // The whole item in one load per wave, a field per lane: its header, table
+  // entries, and everything that depends on them, are then one memory round
+  // trip away instead of three in a row.  With the slots and queries requested
+  // together below, the time before the first tile is that of its ~850
+  // instructions, no longer of a chain of loads: 15 spans over 32k keys (28/4
+  // heads) 75.1 -> 73.2 us, 168 spans of 24 requests 153.7 -> 152.1 us.
+  static_assert(kItemInts > kWave && kItemInts <= 2 * kWave, "two fields per lane");
+  // The kernel arguments in one group of scalar loads, ahead of their uses.
+  asm volatile("" ::"s"(p.items), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.slots), "s"(p.positions), "s"(p.num_queries),
+               "s"(p.num_slots), "s"(p.slots_len), "s"(p.ws_items), "s"(p.hq), "s"(p.hkv), "s"(p.group),
+               "s"(p.pair_chunks), "s"(p.slots64), "s"(p.pool_bytes));
+  const int *item_ptr = p.items + static_cast<long long>(blockIdx.x) * kItemInts;
+  const int item_lane = threadIdx.x % kWave;
+  int item_lo = item_ptr[item_lane];
+  int item_hi = item_ptr[min(kWave + item_lane, kItemInts - 1)];
+  asm volatile("" : "+v"(item_lo), "+v"(item_hi));  // both now: a later wait for one would wait for the slots too
+  auto it = [&](int field) {  // field: wave-uniform
+    const int lo = __builtin_amdgcn_readlane(item_lo, field & (kWave - 1));
+    const int hi = __builtin_amdgcn_readlane(item_hi, field & (kWave - 1));
+    return field < kWave ? lo : hi;
+  };
+  const int kv_off = it(0), kv_begin = it(1), kv_end = it(2), n_tiles = it(3);
+  const int pair_first = it(4), pair_count = it(5);
   // blockIdx.y = (KV head, pair chunk): this workgroup's pairs of the window
   // are [wg_first, wg_end), counted from the item's first tile.
   const int hk = blockIdx.y / p.pair_chunks;
@@ -364,58 +379,14 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   const int col = lane % 32;  // MFMA column of this lane
   const int qc = col % 16;    // query within the column's pair
 
-  // The wave's two pairs; a pair computes when its tile and head exist and its
-  // table entry is sane.
-  struct PairInfo {
-    bool computes;
-    int q_index, q_pos, q_count, partial, stop, hq;
-  };
-  auto pair_info = [&](int pair) {
-    PairInfo r;
-    const int flat = wg_first + pair;  // pair index in the window's tiles
-    const int tile = flat / p.group;
-    const int head = flat - tile * p.group;
-    const bool in_window = flat < wg_end;  // and so tile < n_tiles (checked above)
-    const int *e = it + kItemHeader + kTileInts * (in_window ? tile : 0);
-    r.q_index = e[0];
-    r.q_pos = e[1];
-    r.q_count = e[2];
-    r.partial = e[3];
-    const int needed = e[4];
-    r.hq = hk * p.group + head;
-    r.computes = in_window && r.q_count >= 1 && r.q_count <= kQueries && r.q_index >= 0 &&
-                 static_cast<long long>(r.q_index) + r.q_count <= p.num_queries && r.q_pos >= 0 &&
-                 needed > r.q_pos && (r.partial == -1 || (r.partial >= 0 && r.partial < p.ws_items));
-    r.stop = r.computes ? min(kv_end, needed) : kv_begin;
-    return r;
-  };
-  const PairInfo pair0 = pair_info(2 * wave), pair1 = pair_info(2 * wave + 1);
-  const PairInfo &mine = col < 16 ? pair0 : pair1;
-  const bool wave_computes = pair0.computes || pair1.computes;
-  const int wave_stop = max(pair0.stop, pair1.stop);
-  // Keys below both pairs' lowest query position and stop need no causal mask.
-  int wave_unmasked = kv_end;
-  if (pair0.computes) wave_unmasked = min(wave_unmasked, min(pair0.q_pos, pair0.stop));
-  if (pair1.computes) wave_unmasked = min(wave_unmasked, min(pair1.q_pos, pair1.stop));
-  const bool q_ok = mine.computes && qc < mine.q_count;
-  const int my_pos = q_ok ? p.positions[mine.q_index + qc] : 0;
-  const int my_stop = mine.stop;
-
-  // Keys this workgroup's tiles need.
-  int load_stop = kv_begin;
-  for (int t = wg_first / p.group; t <= (wg_end - 1) / p.group; ++t) {
-    const int *e = it + kItemHeader + kTileInts * t;
-    if (e[2] >= 1) load_stop = max(load_stop, min(kv_end, e[4]));
-  }
-  // B operand of the score MFMAs: the lane's query, dims 16 ks + 8 h .. + 7.
-  frag qf[kKSteps];
-  {
-    const uint16_t *qrow = p.q + (static_cast<long long>(mine.q_index + qc) * p.hq + mine.hq) * D + 8 * h;
-#pragma unroll
-    for (int ks = 0; ks < kKSteps; ++ks) {
-      u32x4 bits = {0u, 0u, 0u, 0u};
-      if (q_ok) bits = *reinterpret_cast<const u32x4 *>(qrow + 16 * ks);
-      qf[ks] = __builtin_bit_cast(frag, bits);
+  // Keys this workgroup's tiles need: the item's (its key end is that of the
+  // window's furthest tile), unless the window takes several workgroups.
+  int load_stop = kv_end;
+  if constexpr (kPairs < kMaxPairs) {
+    load_stop = kv_begin;
+    for (int t = wg_first / p.group; t <= (wg_end - 1) / p.group; ++t) {
+      const int e = kItemHeader + kTileInts * t;
+      if (it(e + 2) >= 1) load_stop = max(load_stop, min(kv_end, it(e + 4)));
     }
   }
 
@@ -437,6 +408,107 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
     g_koff[j] = static_cast<unsigned>(hk * D * 2 + g_kchunk[j] * 16);
     g_voff[j] = static_cast<unsigned>(hk * D * 2 + g_vchunk[j] * 16);
   }
+  // The slots of a chunk of keys, loaded straight into registers: those of
+  // the wave's own gathers of the first kLead tiles, and the thread's first
+  // entries of the slot list.  For the first chunk they are requested here,
+  // together with the queries below, so that the gathers start two memory
+  // round trips after the launch (item, then slots) instead of after the
+  // header, the entries, the queries, the slot list and a barrier in a row.
+  // All loads of a group are unconditional (past the chunk's end its last key
+  // is read again and dropped) and keep the words as they come (an int32 slot
+  // has no high word), so that no wait and no branch separates them.
+  constexpr int kFill = D == 256 ? 4 : 8;  // (registers)
+  unsigned lead_lo[kLead][kGathers], lead_hi[kLead][kGathers], list_lo[kFill], list_hi[kFill];
+  auto load_slots = [&](int chunk_begin, int first, bool lead) __attribute__((always_inline)) {
+    const int last = min(load_stop - chunk_begin, kDmaMaxRange) - 1;
+    const long long base = static_cast<long long>(kv_off) + chunk_begin;
+    auto load = [&](auto read) __attribute__((always_inline)) {
+      if (lead) {
+#pragma unroll
+        for (int t = 0; t < kLead; ++t)
+#pragma unroll
+          for (int j = 0; j < kGathers; ++j)
+            read(min(t * kTile + g_token[j], last), lead_lo[t][j], lead_hi[t][j]);
+      }
+#pragma unroll
+      for (int u = 0; u < kFill; ++u)
+        read(min(first + u * kM32Threads, last), list_lo[u], list_hi[u]);
+    };
+    if (p.slots64) {
+      const u32x2 *slots = static_cast<const u32x2 *>(p.slots) + base;
+      load([&](int i, unsigned &lo, unsigned &hi) __attribute__((always_inline)) {
+        const u32x2 slot = slots[i];
+        lo = slot[0];
+        hi = slot[1];
+      });
+    } else {
+      const unsigned *slots = static_cast<const unsigned *>(p.slots) + base;
+      load([&](int i, unsigned &lo, unsigned &hi) __attribute__((always_inline)) {
+        lo = slots[i];
+        hi = 0u;
+      });
+    }
+  };
+  auto load_first_slots = [&](int chunk_begin) __attribute__((always_inline)) {
+    load_slots(chunk_begin, tid, true);
+  };
+  if (load_stop <= kv_begin) load_stop = kv_begin;  // no keys: no slots, no tiles
+  else
+  load_first_slots(kv_begin);
+
+  // The wave's two pairs; a pair computes when its tile and head exist and its
+  // table entry is sane.
+  struct PairInfo {
+    bool computes;
+    int q_index, q_pos, q_count, partial, stop, hq;
+  };
+  auto pair_info = [&](int pair) {
+    PairInfo r;
+    const int flat = wg_first + pair;  // pair index in the window's tiles
+    const int tile = flat / p.group;
+    const int head = flat - tile * p.group;
+    const bool in_window = flat < wg_end;  // and so tile < n_tiles (checked above)
+    const int e = kItemHeader + kTileInts * (in_window ? tile : 0);
+    r.q_index = it(e);
+    r.q_pos = it(e + 1);
+    r.q_count = it(e + 2);
+    r.partial = it(e + 3);
+    const int needed = it(e + 4);
+    r.hq = hk * p.group + head;
+    r.computes = in_window && r.q_count >= 1 && r.q_count <= kQueries && r.q_index >= 0 &&
+                 static_cast<long long>(r.q_index) + r.q_count <= p.num_queries && r.q_pos >= 0 &&
+                 needed > r.q_pos && (r.partial == -1 || (r.partial >= 0 && r.partial < p.ws_items));
+    r.stop = r.computes ? min(kv_end, needed) : kv_begin;
+    return r;
+  };
+  const PairInfo pair0 = pair_info(2 * wave), pair1 = pair_info(2 * wave + 1);
+  const PairInfo &mine = col < 16 ? pair0 : pair1;
+  const bool wave_computes = pair0.computes || pair1.computes;
+  const int wave_stop = max(pair0.stop, pair1.stop);
+  // Keys below both pairs' lowest query position and stop need no causal mask.
+  int wave_unmasked = kv_end;
+  if (pair0.computes) wave_unmasked = min(wave_unmasked, min(pair0.q_pos, pair0.stop));
+  if (pair1.computes) wave_unmasked = min(wave_unmasked, min(pair1.q_pos, pair1.stop));
+  const bool q_ok = mine.computes && qc < mine.q_count;
+  const int my_stop = mine.stop;
+
+  // B operand of the score MFMAs: the lane's query, dims 16 ks + 8 h .. + 7.
+  frag qf[kKSteps];
+  int my_pos = 0;
+  {
+    u32x4 bits[kKSteps];
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) bits[ks] = u32x4{0u, 0u, 0u, 0u};
+    if (q_ok) {
+      my_pos = p.positions[mine.q_index + qc];
+      const uint16_t *qrow = p.q + (static_cast<long long>(mine.q_index + qc) * p.hq + mine.hq) * D + 8 * h;
+#pragma unroll
+      for (int ks = 0; ks < kKSteps; ++ks) bits[ks] = *reinterpret_cast<const u32x4 *>(qrow + 16 * ks);
+    }
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) qf[ks] = __builtin_bit_cast(frag, bits[ks]);
+  }
+
   const i32x4r k_res = buffer_resource(p.k, p.pool_bytes);
   const i32x4r v_res = buffer_resource(p.v, p.pool_bytes);
   auto gather_slots = [&](int t, int *slots) {
@@ -460,10 +532,13 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
       }
     }
   };
-  auto gather = [&](int t, unsigned char *k_dst, unsigned char *v_dst) {
-    int slots[kGathers];
-    gather_slots(t, slots);
-    gather_from(slots, k_dst, v_dst);
+  // A slot as loaded: valid, and its entry of the slot list.
+  auto slot_valid = [&](unsigned lo, unsigned hi, bool in_range) {
+    return in_range && hi == 0u && lo < static_cast<unsigned>(p.num_slots);  // num_slots < 2^31
+  };
+  auto list_entry = [&](unsigned lo, bool valid) {
+    if constexpr (kOffsets) return static_cast<int>((valid ? lo : 0u) * static_cast<unsigned>(2 * row_stride));
+    else return valid ? static_cast<int>(lo) : -1;
   };
 
   float m = kScoreFloor;
@@ -515,30 +590,41 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   // per chunk the slot list is refilled (the ring drained at the chunk's end
   // and restarted), while the softmax state carries over, so one workgroup
   // takes a key range of any length.
-  for (int chunk_begin = kv_begin; chunk_begin < load_stop; chunk_begin += kDmaMaxRange) {
+  for (int chunk_begin = kv_begin; chunk_begin < load_stop;) {
   const int range = min(load_stop - chunk_begin, kDmaMaxRange);
   const int tiles = (range + kTile - 1) / kTile;
-  if (chunk_begin != kv_begin) __syncthreads();  // every wave is done with the previous chunk's slots and stages
   // Each wave takes whole 64-token tiles (the workgroup is a whole number of
   // waves), so a tile's valid-slot bits are one ballot.
-  for (int i = tid; i < tiles * kTile; i += kM32Threads) {
-    int slot = -1;
-    if (i < range) {
-      const long long s = slot_at(p, static_cast<long long>(kv_off) + chunk_begin + i);
-      if (s >= 0 && s < p.num_slots) slot = static_cast<int>(s);
-    }
-    if constexpr (kOffsets)
-      slot_lds[i] = static_cast<int>(static_cast<unsigned>(slot >= 0 ? slot : 0) * static_cast<unsigned>(2 * row_stride));
-    else
-      slot_lds[i] = slot;
-    const unsigned long long bits = __builtin_amdgcn_ballot_w64(slot >= 0);
-    if (lane == 0) tile_valid[i / kTile] = bits;
-  }
-  __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0): the slots (and, in the first chunk, the queries) are in
-  __syncthreads();
+  auto store_slots = [&](int base) {  // list_lo, list_hi: entries base, base + kM32Threads, ...
 #pragma unroll
-  for (int t = 0; t < kLead; ++t)
-    if (t < tiles) gather(t, k_ring + t * kStageBytes, v_ring + t * kStageBytes);
+    for (int u = 0; u < kFill; ++u) {
+      const int i = base + u * kM32Threads;
+      if (i >= tiles * kTile) break;
+      const bool valid = slot_valid(list_lo[u], list_hi[u], i < range);
+      slot_lds[i] = list_entry(list_lo[u], valid);
+      const unsigned long long bits = __builtin_amdgcn_ballot_w64(valid);
+      if (lane == 0) tile_valid[i / kTile] = bits;
+    }
+  };
+  // The slots (and, in the first chunk, the queries) are in.  The compiler does
+  // not count the gathers issued from here on, so nothing that it waits for in
+  // the tile loop may be left in flight.
+  __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
+  store_slots(tid);
+#pragma unroll
+  for (int t = 0; t < kLead; ++t) {
+    int slots[kGathers];
+#pragma unroll
+    for (int j = 0; j < kGathers; ++j)
+      slots[j] = list_entry(lead_lo[t][j], slot_valid(lead_lo[t][j], lead_hi[t][j], t * kTile + g_token[j] < range));
+    if (t < tiles) gather_from(slots, k_ring + t * kStageBytes, v_ring + t * kStageBytes);
+  }
+  for (int base = tid + kFill * kM32Threads; base < tiles * kTile; base += kFill * kM32Threads) {
+    load_slots(chunk_begin, base, false);
+    store_slots(base);
+  }
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot list is written (the gathers stay in flight)
+  workgroup_barrier();
   static_assert(kStages == 2 || kStages == 4, "the tile loop is unrolled over the ring's stages");
   // One tile; the ring stage (t % kStages) is a compile-time constant, so
   // that the stage offsets of the LDS reads are immediates.
@@ -716,6 +802,10 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
       if (tb + 3 < tiles) tile_step(tb + 3, std::integral_constant<int, 3>{});
     }
   }
+  if (load_stop - chunk_begin <= kDmaMaxRange) break;
+  chunk_begin += kDmaMaxRange;
+  __syncthreads();  // every wave is done with this chunk's slots and stages
+  load_first_slots(chunk_begin);
   }  // key chunks
   // The column's other half (lane l ^ 32) summed the other tokens.
   {

@@ -539,6 +539,19 @@ int ll_repair_attention_plan(const ll_repair_row *rows, int64_t num_rows, int64_
                              int64_t items_capacity, int32_t *combine, int64_t combine_capacity,
                              int32_t *positions, int64_t positions_capacity,
                              ll_repair_attention_plan_info *info);
+/*
+ * The same, with what the choice of the chunk length (split_tokens 0) may know
+ * besides: head_dim (64, 128 or 256; 0: not known), whose workgroups per item
+ * and partial sizes the model then takes and for which chunks below 512 keys
+ * are tried where they fill idle compute units, and workspace_limit, the bytes
+ * of partial results that the plan may need (0: any;
+ * ll_repair_attention_noalloc takes LL_REPAIR_SCRATCH_BYTES).
+ */
+int ll_repair_attention_plan_dim(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_heads,
+                                 int64_t num_kv_heads, int64_t head_dim, int64_t split_tokens,
+                                 int64_t workspace_limit, int32_t *items, int64_t items_capacity,
+                                 int32_t *combine, int64_t combine_capacity, int32_t *positions,
+                                 int64_t positions_capacity, ll_repair_attention_plan_info *info);
 int ll_repair_attention(const ll_repair_attention_args *args, ll_stream_t stream);
 
 /*

@@ -79,6 +79,9 @@ constexpr int kItemHeader = 6;
 constexpr int kTileInts = 5;
 constexpr int kItemInts = kItemHeader + kTileInts * kMaxTiles;  // 86
 constexpr int kCombineInts = 4;
+// Set in an item's pair count and in a combine item's query count: the split
+// results are wide (fp32 outputs), each taking two partial slots.
+constexpr int kWide = 0x100;
 
 int fail(int code, const char *fmt, ...) {
   va_list ap;
@@ -157,10 +160,17 @@ struct F16 {
 // rounding the probabilities to the KV dtype already allows.
 template <int D>
 __host__ __device__ constexpr int partial_floats() { return kQueries * D / 2 + 2 * kQueries; }
+// A wide partial keeps O / l in fp32, [16][D] floats and then (m, l) as above,
+// in the space of two partial slots (16 D + 64 floats per head).  Plans with
+// chunks below 512 keys use them: such a chunk may split what one workgroup
+// would otherwise keep in fp32 from end to end, and the few partials of so
+// small a plan cost nothing (2,048 keys: 17.3 us either way).
 template <int D>
-__device__ inline float *partial_block(const AttnParams &p, int partial, int h) {
-  return p.ws + (static_cast<long long>(partial) * p.hq + h) * partial_floats<D>();
+__device__ inline float *partial_block(const AttnParams &p, int partial, int h, bool wide) {
+  return p.ws + (static_cast<long long>(partial) * p.hq + (wide ? 2 * h : h)) * partial_floats<D>();
 }
+template <int D>
+__device__ inline int partial_sums(bool wide) { return wide ? kQueries * D : kQueries * D / 2; }  // (m, l) offset
 
 // v_permlane32_swap a, b exchanges the upper half of a with the lower half of
 // b: from two copies of x it leaves (x[l], x[l ^ 32]) in the lane, up to
@@ -357,7 +367,8 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
     return field < kWave ? lo : hi;
   };
   const int kv_off = it(0), kv_begin = it(1), kv_end = it(2), n_tiles = it(3);
-  const int pair_first = it(4), pair_count = it(5);
+  const int pair_first = it(4), pair_count = it(5) & (kWide - 1);
+  const bool wide = (it(5) & kWide) != 0;
   // blockIdx.y = (KV head, pair chunk): this workgroup's pairs of the window
   // are [wg_first, wg_end), counted from the item's first tile.
   const int hk = blockIdx.y / p.pair_chunks;
@@ -477,7 +488,7 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
     r.hq = hk * p.group + head;
     r.computes = in_window && r.q_count >= 1 && r.q_count <= kQueries && r.q_index >= 0 &&
                  static_cast<long long>(r.q_index) + r.q_count <= p.num_queries && r.q_pos >= 0 &&
-                 needed > r.q_pos && (r.partial == -1 || (r.partial >= 0 && r.partial < p.ws_items));
+                 needed > r.q_pos && (r.partial == -1 || (r.partial >= 0 && r.partial < p.ws_items - (wide ? 1 : 0)));
     r.stop = r.computes ? min(kv_end, needed) : kv_begin;
     return r;
   };
@@ -818,7 +829,24 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   // Register r of dim block b holds dim 32 b + 8 (r / 4) + 4 h + r % 4.
   if (!q_ok) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  float *block = mine.partial < 0 ? nullptr : partial_block<D>(p, mine.partial, mine.hq);
+  float *block = mine.partial < 0 ? nullptr : partial_block<D>(p, mine.partial, mine.hq, wide);
+  if (block != nullptr && h == 0) {
+    block[partial_sums<D>(wide) + 2 * qc] = m * scale_log2;
+    block[partial_sums<D>(wide) + 2 * qc + 1] = l;
+  }
+  if (block != nullptr && wide) {
+    float *dst = block + qc * D + 4 * h;
+#pragma unroll
+    for (int b = 0; b < kDimBlocks; ++b)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        f32x4 row;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) row[e] = o[b][4 * rr + e] * inv;
+        *reinterpret_cast<f32x4 *>(dst + 32 * b + 8 * rr) = row;
+      }
+    return;
+  }
   uint16_t *dst = block == nullptr
                       ? p.out + (static_cast<long long>(mine.q_index + qc) * p.hq + mine.hq) * D + 4 * h
                       : reinterpret_cast<uint16_t *>(block) + qc * D + 4 * h;
@@ -831,48 +859,34 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
       packed[1] = E::pack(o[b][4 * rr + 2] * inv, o[b][4 * rr + 3] * inv);
       *reinterpret_cast<u32x2 *>(dst + 32 * b + 8 * rr) = packed;
     }
-  if (block != nullptr && h == 0) {
-    block[kQueries * D / 2 + 2 * qc] = m * scale_log2;
-    block[kQueries * D / 2 + 2 * qc + 1] = l;
-  }
 }
 
-// Merges the split partial results of one 16-query tile: workgroup (combine
-// item, query head); thread = (query, 1/16 of the dims).
-template <int D, typename E>
-__global__ void __launch_bounds__(256) repair_combine_kernel(const AttnParams p) {
+// The sum of the partials of one query and 1/16 of the dims (in acc), and of
+// their weights.  One pass in batches of kBatch partials whose loads are all in flight
+// together; the running maximum rescales what is summed when a batch raises
+// it.  A partial's weight is its sum l times 2^(m - max): its normalised
+// output O / l then contributes exactly O.
+template <int D, typename E, bool kWidePartials>
+__device__ inline float merge_partials(const AttnParams &p, int first, int count, int h, int c, int part,
+                                       f32x4 *acc) {
   constexpr int kPer = D / 16;
-  const int *ci = p.combine + static_cast<long long>(blockIdx.x) * kCombineInts;
-  const int q_index = ci[0], q_count = ci[1], first = ci[2], count = ci[3];
-  if (q_count < 1 || q_count > kQueries || q_index < 0 ||
-      static_cast<long long>(q_index) + q_count > p.num_queries || first < 0 || count < 1 ||
-      static_cast<long long>(first) + count > p.ws_items)
-    return;
-  const int h = blockIdx.y;
-  const int c = threadIdx.x / 16;
-  const int part = threadIdx.x % 16;
-  if (c >= q_count) return;
-  // One pass in batches of kBatch partials whose loads are all in flight
-  // together; the running maximum rescales what is summed when a batch
-  // raises it.  A partial's weight is its sum l times 2^(m - max): its
-  // normalised output O / l then contributes exactly O.
   constexpr int kBatch = 8;
+  typedef std::conditional_t<kWidePartials, f32x4, u32x2> Quad;  // four values of a partial's row
   float run_max = -INFINITY;
   float total = 0.f;
-  f32x4 acc[kPer / 4];
-#pragma unroll
-  for (int d = 0; d < kPer / 4; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < count; s0 += kBatch) {
     float ms[kBatch], ls[kBatch];
-    u32x2 rows[kBatch][kPer / 4];  // kPer 16-bit values: kPer / 4 pairs of words
+    Quad rows[kBatch][kPer / 4];
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int s = min(s0 + i, count - 1);  // past the end: the last partial again, unused
-      const float *block = partial_block<D>(p, first + s, h);
-      ms[i] = block[kQueries * D / 2 + 2 * c];
-      ls[i] = block[kQueries * D / 2 + 2 * c + 1];
-      const u32x2 *row = reinterpret_cast<const u32x2 *>(reinterpret_cast<const uint16_t *>(block) + c * D +
-                                                         part * kPer);
+      const float *block = partial_block<D>(p, first + (kWidePartials ? 2 * s : s), h, kWidePartials);
+      ms[i] = block[partial_sums<D>(kWidePartials) + 2 * c];
+      ls[i] = block[partial_sums<D>(kWidePartials) + 2 * c + 1];
+      const Quad *row = kWidePartials
+                            ? reinterpret_cast<const Quad *>(block + c * D + part * kPer)
+                            : reinterpret_cast<const Quad *>(reinterpret_cast<const uint16_t *>(block) + c * D +
+                                                             part * kPer);
 #pragma unroll
       for (int d = 0; d < kPer / 4; ++d) rows[i][d] = row[d];
     }
@@ -893,12 +907,40 @@ __global__ void __launch_bounds__(256) repair_combine_kernel(const AttnParams p)
       total += w;
 #pragma unroll
       for (int d = 0; d < kPer / 4; ++d) {  // values 4 d .. 4 d + 3
-        const f32x2 v0 = E::unpack(rows[i][d][0]);
-        const f32x2 v1 = E::unpack(rows[i][d][1]);
-        acc[d] += w * f32x4{v0[0], v0[1], v1[0], v1[1]};
+        if constexpr (kWidePartials) {
+          acc[d] += w * rows[i][d];
+        } else {
+          const f32x2 v0 = E::unpack(rows[i][d][0]);
+          const f32x2 v1 = E::unpack(rows[i][d][1]);
+          acc[d] += w * f32x4{v0[0], v0[1], v1[0], v1[1]};
+        }
       }
     }
   }
+  return total;
+}
+
+// Merges the split partial results of one 16-query tile: workgroup (combine
+// item, query head); thread = (query, 1/16 of the dims).
+template <int D, typename E>
+__global__ void __launch_bounds__(256) repair_combine_kernel(const AttnParams p) {
+  constexpr int kPer = D / 16;
+  const int *ci = p.combine + static_cast<long long>(blockIdx.x) * kCombineInts;
+  const int q_index = ci[0], q_count = ci[1] & (kWide - 1), first = ci[2], count = ci[3];
+  const bool wide = (ci[1] & kWide) != 0;
+  if (q_count < 1 || q_count > kQueries || q_index < 0 ||
+      static_cast<long long>(q_index) + q_count > p.num_queries || first < 0 || count < 1 ||
+      static_cast<long long>(first) + (wide ? 2ll : 1ll) * count > p.ws_items)
+    return;
+  const int h = blockIdx.y;
+  const int c = threadIdx.x / 16;
+  const int part = threadIdx.x % 16;
+  if (c >= q_count) return;
+  f32x4 acc[kPer / 4];
+#pragma unroll
+  for (int d = 0; d < kPer / 4; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float total = wide ? merge_partials<D, E, true>(p, first, count, h, c, part, acc)
+                           : merge_partials<D, E, false>(p, first, count, h, c, part, acc);
   const float inv = total > 0.f ? 1.f / total : 0.f;
   uint16_t *dst = p.out + (static_cast<long long>(q_index + c) * p.hq + h) * D + part * kPer;
   uint32_t packed[kPer / 2];
@@ -919,12 +961,19 @@ constexpr int kComputeUnits = 256;          // MI355X
 constexpr double kItemOverheadTiles = 3.0;  // slots, queries, write-out
 constexpr double kPartialBytesPerTile = 12e6;  // partial results the combine reads in one tile's time
 constexpr double kCombineLaunchTiles = 2.0;
+// The combine merges a query tile's partials one batch after another: at
+// 2,048 keys it takes 5 us for 4 chunks, 7 us for 16 (0.1-0.17 us each), and
+// 45 us for 512 of a single span over 32k keys.
+constexpr double kCombineChunkTiles = 0.05;
 constexpr int64_t kRefillTiles = 2;  // an item's slot-list refill (every kDmaMaxRange keys): drain and restart
 // A plan whose cost provably exceeds `beat` returns early with a lower bound
 // of its cost (still above `beat`).
+// `workgroups` is a work item's workgroups, `partial_bytes` those of one partial
+// result (all query heads).  A plan whose partials need more than
+// `workspace_limit` bytes (0: no limit) costs HUGE_VAL.
 template <typename Groups>
-double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t num_q_heads, double beat,
-                          Groups &&groups) {
+double plan_cost_estimate(int64_t split, int64_t workgroups, int64_t partial_bytes, int64_t workspace_limit,
+                          double beat, Groups &&groups) {
   // A group of `needed` keys makes needed / split full chunks and one shorter
   // one.  Costs are whole numbers of tiles, so their sums are exact in double
   // and do not depend on the order they are added in.
@@ -933,11 +982,12 @@ double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t num_q_hea
            kRefillTiles * ((keys - 1) / kDmaMaxRange);
   };
   const double full_cost = static_cast<double>(tiles_of(split));
-  int64_t partials = 0, count = 0;
+  int64_t partials = 0, count = 0, most_chunks = 0;
   double total = 0.0, longest = 0.0;
   groups([&](int64_t needed, int64_t group_partials) {
     const int64_t full = needed / split, rest = needed - full * split;
     count += full + (rest > 0);
+    most_chunks = full + (rest > 0) > most_chunks ? full + (rest > 0) : most_chunks;
     total += static_cast<double>(full) * full_cost;
     if (full > 0) longest = full_cost > longest ? full_cost : longest;
     if (rest > 0) {
@@ -948,18 +998,20 @@ double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t num_q_hea
     partials += group_partials;
   });
   double combine_cost = 0.0;
-  if (partials > 0)  // 16 queries' 16-bit outputs (head dim 128) and fp32 (max, sum) per partial and head
-    combine_cost = kCombineLaunchTiles + static_cast<double>(partials) * num_q_heads *
-                                             (kQueries * 128 * 2 + 2 * kQueries * 4) / kPartialBytesPerTile;
+  const double bytes = static_cast<double>(partials) * static_cast<double>(partial_bytes);
+  if (workspace_limit > 0 && bytes > static_cast<double>(workspace_limit)) return HUGE_VAL;
+  if (partials > 0)
+    combine_cost = kCombineLaunchTiles + kCombineChunkTiles * static_cast<double>(most_chunks) +
+                   bytes / kPartialBytesPerTile;
   if (count == 0) return combine_cost;
-  if (count * num_kv_heads > 8 * kComputeUnits) {
+  if (count * workgroups > 8 * kComputeUnits) {
     // Many rounds: the last one's imbalance is small against the total; it
     // leaves about half of the longest item to run alone.
-    return total * num_kv_heads / kComputeUnits + 0.5 * longest + combine_cost;
+    return total * workgroups / kComputeUnits + 0.5 * longest + combine_cost;
   }
   // No schedule ends before its longest item or before the CUs have run
   // every item's work.
-  const double spread = total * static_cast<double>(num_kv_heads) / kComputeUnits;
+  const double spread = total * static_cast<double>(workgroups) / kComputeUnits;
   const double bound = (longest > spread ? longest : spread) + combine_cost;
   if (bound > beat) return bound;
   double makespan = 0.0;
@@ -977,13 +1029,13 @@ double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t num_q_hea
   item_cost.reserve(static_cast<size_t>(count));
   for (int64_t c = max_cost; c > 0; --c) item_cost.insert(item_cost.end(), static_cast<size_t>(cost_count[c]), c);
   const int64_t n = static_cast<int64_t>(item_cost.size());
-  if (n * num_kv_heads <= 2 * kComputeUnits) {
+  if (n * workgroups <= 2 * kComputeUnits) {
     // At most two rounds: the workgroups beyond the first 256 start when the
     // first round has ended (measured on c2: its 4 extra workgroups started
     // 72 us into an 82 us kernel, not when the first short items freed their
     // CUs), so the rounds' longest items add up.
     int64_t second = 0;
-    for (int64_t g = kComputeUnits; g < n * num_kv_heads; ++g) {
+    for (int64_t g = kComputeUnits; g < n * workgroups; ++g) {
       const int64_t cost = item_cost[static_cast<size_t>(g % n)];  // grid order: items, then KV heads
       second = cost > second ? cost : second;
     }
@@ -994,7 +1046,7 @@ double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t num_q_hea
     // counted by free time and the earliest is found by moving forward.
     std::vector<int32_t> free_from(1, kComputeUnits);
     int64_t now = 0, last_end = 0;
-    for (int64_t h = 0; h < num_kv_heads; ++h) {
+    for (int64_t h = 0; h < workgroups; ++h) {
       for (const int64_t cost : item_cost) {
         while (free_from[static_cast<size_t>(now)] == 0) ++now;
         --free_from[static_cast<size_t>(now)];
@@ -1176,14 +1228,15 @@ namespace {
 // same rows and heads then compute it once.
 struct RepairPlan {
   std::vector<ll_repair_row> rows;
-  int64_t num_q_heads = -1, num_kv_heads = -1, split_in = -1;
+  int64_t num_q_heads = -1, num_kv_heads = -1, head_dim = -1, split_in = -1, workspace_limit = -1;
   std::vector<int32_t> items, combine, positions;
   std::vector<int32_t> sorted;  // reordering space for the items
   ll_repair_attention_plan_info info{};
 };
 
+// head_dim 0: not known (planned as 128, with chunks of at least 512 keys).
 int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_heads, int64_t num_kv_heads,
-                 int64_t split_tokens, RepairPlan &out) {
+                 int64_t head_dim, int64_t split_tokens, int64_t workspace_limit, RepairPlan &out) {
   constexpr int64_t kIntMax = 0x7fffffff;
   const int64_t group = num_q_heads / num_kv_heads;
   // 16-query tiles in row order.  Consecutive rows of one request (the next
@@ -1282,6 +1335,9 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
       needed = tiles[t].needed > needed ? tiles[t].needed : needed;
     window_keys[k] = needed;
   }
+  const int64_t dim = head_dim > 0 ? head_dim : 128;
+  const int64_t workgroups = num_kv_heads * (kMaxPairs / max_pairs(static_cast<int>(dim)));
+  const int64_t partial_bytes = num_q_heads * (kQueries * dim * 2 + 2 * kQueries * 4);  // of one partial slot
   int64_t split = split_tokens;
   if (split == 0) {
     // Pick the chunk length whose plan finishes first on a model of the
@@ -1289,14 +1345,14 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     // workgroups dispatched in grid order to the first free CU, each costing
     // its key tiles plus a fixed overhead, then the combine pass reading every
     // partial result.  Few long chunks leave CUs idle in the last round; many
-    // short ones add overhead and partials.  A coarse pass over lengths from
-    // 512 to the maximum, then every multiple of the key tile within 256 of
+    // short ones add overhead and partials.  A coarse pass over lengths up to
+    // the maximum, then every multiple of the key tile within 256 of
     // the best: one tile more per item can save a round (c2: 2,112 keys make
     // 64 items, one round of 4 KV heads on 256 CUs, where 2,048 make 65).
     double best = -1.0;
     auto estimate = [&](int64_t candidate) {
       const double beat = best < 0.0 ? HUGE_VAL : best;
-      return plan_cost_estimate(candidate, num_kv_heads, num_q_heads, beat, [&](auto &&visit) {
+      return plan_cost_estimate(candidate, workgroups, partial_bytes, workspace_limit, beat, [&](auto &&visit) {
         int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
         for (size_t k = 0; k < windows.size(); ++k) {
           const Window &w = windows[k];
@@ -1317,7 +1373,17 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     int64_t longest = kTile;
     for (const int64_t keys : window_keys) longest = keys > longest ? keys : longest;
     longest = (longest + kTile - 1) / kTile * kTile;
-    std::vector<int64_t> candidates(std::begin(kCoarse), std::end(kCoarse));
+    // Lengths below 512 where 512-key chunks leave compute units idle: three
+    // 8-row spans over 2,048 keys (28/4 heads) take 24.2 us in 16 workgroups of
+    // 512 keys and 16.2 us in 52 of 128; where 512-key chunks fill the device,
+    // shorter ones only add rounds (15 spans over 32k keys: 108 us at 512, 122
+    // at 384, 234 at 128).
+    std::vector<int64_t> candidates;
+    int64_t items_512 = 0;
+    for (const int64_t keys : window_keys) items_512 += (keys + 511) / 512;
+    const bool small = head_dim > 0 && items_512 * workgroups < kComputeUnits;
+    if (small) candidates = {64, 128, 192, 256, 320, 384, 448};
+    candidates.insert(candidates.end(), std::begin(kCoarse), std::end(kCoarse));
     for (int64_t c = kCoarse[16] * 3 / 2 / kTile * kTile; c < longest; c = c * 3 / 2 / kTile * kTile)
       candidates.push_back(c);
     if (longest > kCoarse[16]) candidates.push_back(longest);
@@ -1330,7 +1396,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     }
     const int64_t coarse = split;
     for (int64_t candidate = coarse - 256; candidate <= coarse + 256; candidate += kTile) {
-      if (candidate < 512 || candidate == coarse) continue;
+      if (candidate < (small ? kTile : 512) || candidate == coarse) continue;
       const double cost = estimate(candidate);
       if (cost < best || (cost == best && candidate > split)) {
         best = cost;
@@ -1345,13 +1411,24 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
   out.combine.clear();
   for (int64_t t = 0; t < n_tiles; ++t) {
     chunks[t] = (tiles[t].needed + split - 1) / split;
+    n_partial += chunks[t] > 1 ? chunks[t] : 0;
+  }
+  // Wide partials, which take two slots each, for chunks below 512 keys (where
+  // the workspace limit allows them).
+  const bool wide = head_dim > 0 && split < 512 && n_partial > 0 && n_partial <= kIntMax / 2 &&
+                    (workspace_limit == 0 ||
+                     static_cast<double>(2 * n_partial) * static_cast<double>(partial_bytes) <=
+                         static_cast<double>(workspace_limit));
+  const int64_t slots_per_partial = wide ? 2 : 1;
+  n_partial = 0;
+  for (int64_t t = 0; t < n_tiles; ++t) {
     if (chunks[t] < 2) continue;
     out.combine.push_back(static_cast<int32_t>(tiles[t].q_index));
-    out.combine.push_back(static_cast<int32_t>(tiles[t].count));
+    out.combine.push_back(static_cast<int32_t>(tiles[t].count | (wide ? kWide : 0)));
     out.combine.push_back(static_cast<int32_t>(n_partial));
     out.combine.push_back(static_cast<int32_t>(chunks[t]));
     base[t] = n_partial;
-    n_partial += chunks[t];
+    n_partial += slots_per_partial * chunks[t];
     ++n_combine;
   }
   for (const int64_t needed : window_keys) n_items += (needed + split - 1) / split;
@@ -1370,14 +1447,14 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
       it[2] = static_cast<int32_t>((s + 1) * split < needed ? (s + 1) * split : needed);
       it[3] = static_cast<int32_t>(w.last - w.first);
       it[4] = static_cast<int32_t>(w.pair_first);
-      it[5] = static_cast<int32_t>(w.pair_count);
+      it[5] = static_cast<int32_t>(w.pair_count | (wide ? kWide : 0));
       for (int64_t t = w.first; t < w.last; ++t) {
         int32_t *e = it + kItemHeader + kTileInts * (t - w.first);
         e[0] = static_cast<int32_t>(tiles[t].q_index);
         e[1] = static_cast<int32_t>(tiles[t].pos);
         const bool present = s < chunks[t];  // this chunk holds keys the tile sees
         e[2] = present ? static_cast<int32_t>(tiles[t].count) : 0;
-        e[3] = !present || chunks[t] == 1 ? -1 : static_cast<int32_t>(base[t] + s);
+        e[3] = !present || chunks[t] == 1 ? -1 : static_cast<int32_t>(base[t] + slots_per_partial * s);
         e[4] = static_cast<int32_t>(tiles[t].needed);
       }
     }
@@ -1423,6 +1500,16 @@ int ll_repair_attention_plan(const ll_repair_row *rows, int64_t num_rows, int64_
                              int64_t items_capacity, int32_t *combine, int64_t combine_capacity,
                              int32_t *positions, int64_t positions_capacity,
                              ll_repair_attention_plan_info *info) {
+  return ll_repair_attention_plan_dim(rows, num_rows, num_q_heads, num_kv_heads, 0, split_tokens, 0, items,
+                                      items_capacity, combine, combine_capacity, positions, positions_capacity,
+                                      info);
+}
+
+int ll_repair_attention_plan_dim(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_heads,
+                                 int64_t num_kv_heads, int64_t head_dim, int64_t split_tokens,
+                                 int64_t workspace_limit, int32_t *items, int64_t items_capacity,
+                                 int32_t *combine, int64_t combine_capacity, int32_t *positions,
+                                 int64_t positions_capacity, ll_repair_attention_plan_info *info) {
   if (info == nullptr) return fail(LL_ERR_INVALID_ARGUMENT, "info is NULL");
   if (num_rows < 0 || (num_rows > 0 && rows == nullptr))
     return fail(LL_ERR_INVALID_ARGUMENT, "rows must be a host array of num_rows >= 0 entries");
@@ -1433,19 +1520,26 @@ int ll_repair_attention_plan(const ll_repair_row *rows, int64_t num_rows, int64_
                 kTile);
   if (num_q_heads > 65535)
     return fail(LL_ERR_KV_HEAD_LAYOUT_MISMATCH, "num_q_heads must be at most 65535");
+  if (head_dim != 0 && head_dim != 64 && head_dim != 128 && head_dim != 256)
+    return fail(LL_ERR_HEAD_DIMENSION_OUT_OF_RANGE, "head_dim must be 64, 128 or 256 (or 0: not known)");
+  if (workspace_limit < 0) return fail(LL_ERR_INVALID_ARGUMENT, "workspace_limit is negative");
   thread_local RepairPlan kept;
   const bool same_rows =
       static_cast<int64_t>(kept.rows.size()) == num_rows && kept.num_q_heads == num_q_heads &&
-      kept.num_kv_heads == num_kv_heads &&
+      kept.num_kv_heads == num_kv_heads && kept.head_dim == head_dim &&
+      kept.workspace_limit == workspace_limit &&
       (split_tokens == kept.split_in || split_tokens == kept.info.split_tokens) &&
       (num_rows == 0 || memcmp(kept.rows.data(), rows, static_cast<size_t>(num_rows) * sizeof(ll_repair_row)) == 0);
   if (!same_rows) {
     kept.num_q_heads = -1;  // invalid until computed
-    const int rc = compute_plan(rows, num_rows, num_q_heads, num_kv_heads, split_tokens, kept);
+    const int rc = compute_plan(rows, num_rows, num_q_heads, num_kv_heads, head_dim, split_tokens,
+                                workspace_limit, kept);
     if (rc != LL_OK) return rc;
     kept.rows.assign(rows, rows + num_rows);
     kept.num_q_heads = num_q_heads;
     kept.num_kv_heads = num_kv_heads;
+    kept.head_dim = head_dim;
+    kept.workspace_limit = workspace_limit;
     kept.split_in = split_tokens;
   }
   const ll_repair_attention_plan_info &plan = kept.info;

@@ -65,6 +65,7 @@ EXPORTED_SYMBOLS = (
     "ll_order_link_maps",
     "ll_order_maps_args_size",
     "ll_repair_attention_plan",
+    "ll_repair_attention_plan_dim",
     "ll_repair_attention",
     "ll_repair_attention_args_size",
     "ll_repair_attention_noalloc",
@@ -384,6 +385,9 @@ def load_library() -> ctypes.CDLL:
         lib.ll_repair_attention_plan.argtypes = [_ptr, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64,
                                                  _ptr, _i64, ctypes.POINTER(RepairPlanInfo)]
         lib.ll_repair_attention_plan.restype = ctypes.c_int
+        lib.ll_repair_attention_plan_dim.argtypes = [_ptr, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr,
+                                                     _i64, _ptr, _i64, ctypes.POINTER(RepairPlanInfo)]
+        lib.ll_repair_attention_plan_dim.restype = ctypes.c_int
         lib.ll_repair_attention.argtypes = [ctypes.POINTER(RepairAttentionArgs), _ptr]
         lib.ll_repair_attention.restype = ctypes.c_int
         lib.ll_repair_attention_args_size.argtypes = []
@@ -460,9 +464,12 @@ def order_link_maps(args: OrderMapsArgs, stream: int) -> None:
     _check(load_library().ll_order_link_maps(ctypes.byref(args), _ptr(int(stream))))
 
 
-def repair_attention_plan(rows, num_q_heads: int, num_kv_heads: int, split_tokens: int = 0):
+def repair_attention_plan(rows, num_q_heads: int, num_kv_heads: int, split_tokens: int = 0, head_dim: int = 0,
+                          workspace_limit: int = 0):
     """Host planning: returns (items int32 [n, 86], combine int32 [m, 4],
-    positions int32 [num_queries], info)."""
+    positions int32 [num_queries], info).  ``head_dim`` (0: not known) and
+    ``workspace_limit`` (bytes of partial results, 0: none) guide the choice
+    of the chunk length."""
 
     import numpy as np
 
@@ -470,20 +477,21 @@ def repair_attention_plan(rows, num_q_heads: int, num_kv_heads: int, split_token
     lib = load_library()
     info = RepairPlanInfo()
     rows_ptr = rows.ctypes.data if rows.size else None
-    _check(lib.ll_repair_attention_plan(rows_ptr, rows.shape[0], int(num_q_heads), int(num_kv_heads),
-                                        int(split_tokens), None, 0, None, 0, None, 0, ctypes.byref(info)))
+    _check(lib.ll_repair_attention_plan_dim(rows_ptr, rows.shape[0], int(num_q_heads), int(num_kv_heads),
+                                            int(head_dim), int(split_tokens), int(workspace_limit), None, 0, None, 0,
+                                            None, 0, ctypes.byref(info)))
     items = np.empty((info.num_items, REPAIR_ITEM_INTS), dtype=np.int32)
     combine = np.empty((info.num_combine, REPAIR_COMBINE_INTS), dtype=np.int32)
     positions = np.empty(info.num_queries, dtype=np.int32)
     # The sizing call chose the chunk length: the filling call takes it as
     # given instead of searching again (same plan, half the host time).
     chosen = int(info.split_tokens)
-    _check(lib.ll_repair_attention_plan(rows_ptr, rows.shape[0], int(num_q_heads), int(num_kv_heads),
-                                        chosen, items.ctypes.data if items.size else None,
-                                        info.num_items,
-                                        combine.ctypes.data if combine.size else None, info.num_combine,
-                                        positions.ctypes.data if positions.size else None, positions.size,
-                                        ctypes.byref(info)))
+    _check(lib.ll_repair_attention_plan_dim(rows_ptr, rows.shape[0], int(num_q_heads), int(num_kv_heads),
+                                            int(head_dim), chosen, int(workspace_limit),
+                                            items.ctypes.data if items.size else None, info.num_items,
+                                            combine.ctypes.data if combine.size else None, info.num_combine,
+                                            positions.ctypes.data if positions.size else None, positions.size,
+                                            ctypes.byref(info)))
     return items, combine, positions, info
 
 

@@ -127,8 +127,12 @@ class RepairAttentionPlan:
                 raise SparseRepairAttentionError("slot_ids contains invalid KV slots")
         self.kv_slots = table
         self.rows = rows
-        items, combine, positions, info = _native.repair_attention_plan(rows, self.num_q_heads,
-                                                                        self.num_kv_heads, split_tokens)
+        self.allocation_free = bool(allocation_free)
+        items, combine, positions, info = _native.repair_attention_plan(
+            rows, self.num_q_heads, self.num_kv_heads, split_tokens,
+            # (a head dim that run() will refuse still plans)
+            head_dim=self.head_dim if self.head_dim in (64, 128, 256) else 0,
+            workspace_limit=_native.repair_scratch_bytes() if self.allocation_free else 0)
         self.info = {"num_items": int(info.num_items), "num_combine": int(info.num_combine),
                      "workspace_items": int(info.workspace_items), "split_tokens": int(info.split_tokens)}
         packed = np.concatenate((items.reshape(-1), combine.reshape(-1), positions)).astype(np.int32)
@@ -137,7 +141,6 @@ class RepairAttentionPlan:
         self.combine = self._tables[items.size : items.size + combine.size]
         self.positions = self._tables[items.size + combine.size :]
         per_item = self.num_q_heads * (8 * self.head_dim + 32)  # 16 x head_dim 16-bit values, 16 (m, l) pairs
-        self.allocation_free = bool(allocation_free)
         self.workspace = (torch.empty(info.workspace_items * per_item, dtype=torch.float32, device=device)
                           if info.workspace_items and not self.allocation_free else None)
 

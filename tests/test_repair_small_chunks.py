@@ -1,0 +1,136 @@
+"""Plans that know the head dim: chunks below 512 keys, wide (fp32) partials,
+the workspace limit, and the two workgroups per window of head dim 256."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from legolink_amd import _native
+from legolink_amd.repair_attention import RepairAttentionPlan
+
+WIDE = 0x100
+
+
+def _rows(context, spans, rows):
+    step = context // (spans + 1)
+    starts = [min(step * (i + 1), context - rows) for i in range(spans)]
+    return np.array([(i * rows, s, rows, 0) for i, s in enumerate(starts)], dtype=np.int64)
+
+
+def _slot_bytes(heads, dim):
+    return heads * (16 * dim * 2 + 128)
+
+
+@pytest.mark.parametrize("context,spans,rows,heads,dim", [
+    (2048, 3, 8, (28, 4), 128), (600, 1, 1, (8, 8), 64), (1000, 5, 16, (64, 8), 256), (4096, 8, 16, (32, 1), 128),
+])
+def test_short_chunks_fill_idle_compute_units_with_wide_partials(context, spans, rows, heads, dim):
+    table = _rows(context, spans, rows)
+    items, combine, positions, info = _native.repair_attention_plan(table, *heads, 0, head_dim=dim)
+    assert info.split_tokens < 512 and info.split_tokens % 64 == 0 and info.num_combine > 0
+    assert (items[:, 5] & WIDE).all() and (combine[:, 1] & WIDE).all()
+    # Every (tile, chunk) has an even slot of its own, two slots wide, inside the workspace.
+    expected = set()
+    for first, count in combine[:, 2:].tolist():
+        expected |= set(range(first, first + 2 * count, 2))
+    assert len(expected) == int(combine[:, 3].sum()) and info.workspace_items == 2 * len(expected)
+    H, T = _native.REPAIR_ITEM_HEADER, _native.REPAIR_TILE_INTS
+    used = set()
+    for item in items.tolist():
+        used |= {item[H + T * t + 3] for t in range(item[3]) if item[H + T * t + 2] > 0} - {-1}
+    assert used == expected
+    # The same plan again with the chosen length given, and the plain entry's
+    # plan (head dim not known): at least 512 keys per chunk, no flag.
+    again = _native.repair_attention_plan(table, *heads, int(info.split_tokens), head_dim=dim)
+    assert np.array_equal(again[0], items) and np.array_equal(again[1], combine)
+    plain = _native.repair_attention_plan(table, *heads, 0)
+    assert plain[3].split_tokens >= 512 and not (plain[0][:, 5] & WIDE).any()
+
+
+def test_chunks_stay_at_512_where_they_fill_the_device():
+    table = _rows(32768, 15, 16)
+    assert _native.repair_attention_plan(table, 28, 4, 0, head_dim=128)[3].split_tokens >= 512
+
+
+@pytest.mark.parametrize("context,spans,rows", [(16384, 15, 16), (8192, 7, 16)])
+def test_head_dim_256_plans_one_round_of_its_two_workgroups_per_window(context, spans, rows):
+    items, _, _, info = _native.repair_attention_plan(_rows(context, spans, rows), 8, 4, 0, head_dim=256)
+    assert info.num_items * 4 * 2 <= 256
+
+
+def test_a_workspace_limit_bounds_the_partials():
+    """Whatever the limit, the plan's partials fit it; the limit of the
+    allocation-free entry is the library's scratch array."""
+
+    table = _rows(32768, 3, 16)
+    for limit in (0, 64 << 20, 8 << 20, 1 << 20, 1):
+        info = _native.repair_attention_plan(table, 64, 8, 0, head_dim=256, workspace_limit=limit)[3]
+        assert limit == 0 or info.workspace_items * _slot_bytes(64, 256) <= limit
+    slots = torch.arange(32768)
+    plan = RepairAttentionPlan([(slots, 32000, 32016)], num_q_heads=512, num_kv_heads=2, head_dim=256,
+                               allocation_free=True)
+    assert plan.info["workspace_items"] * _slot_bytes(512, 256) <= _native.repair_scratch_bytes()
+    # A given length whose 16-bit partials fit the limit is not widened past it.
+    limit = 48 << 20
+    narrow = _native.repair_attention_plan(_rows(16384, 2, 16), 28, 4, 64, head_dim=128, workspace_limit=limit)[3]
+    wide = _native.repair_attention_plan(_rows(16384, 2, 16), 28, 4, 64, head_dim=128)[3]
+    assert narrow.workspace_items * 2 == wide.workspace_items
+    assert narrow.workspace_items * _slot_bytes(28, 128) <= limit < wide.workspace_items * _slot_bytes(28, 128)
+
+
+def test_bad_head_dims_and_limits_are_refused():
+    table = _rows(1000, 1, 8)
+    with pytest.raises(_native.NativeCallError):
+        _native.repair_attention_plan(table, 8, 4, 0, head_dim=96)
+    with pytest.raises(_native.NativeCallError):
+        _native.repair_attention_plan(table, 8, 4, 0, head_dim=128, workspace_limit=-1)
+    # A plan object still takes any head dim (run() refuses it).
+    RepairAttentionPlan([(torch.arange(1000), 1, 9)], num_q_heads=8, num_kv_heads=4, head_dim=96)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("context,spans,rows,heads,dim", [
+    (2048, 3, 8, (28, 4), 128), (513, 2, 17, (8, 8), 64), (1000, 5, 1, (12, 4), 256), (700, 1, 33, (32, 1), 128),
+    (4100, 6, 16, (7, 1), 64), (1471, 4, 16, (64, 8), 256),
+])
+def test_short_chunks_are_as_exact_as_whole_ranges(gpu_device, context, spans, rows, heads, dim, dtype):
+    """Against fp64: within the bound of the probabilities' rounding (half an
+    ulp of each, 2^-8 of weighted |V| with its sum) and the output's (2^-9);
+    wide partials add fp32 terms only.  The error is that of the same run with
+    every range whole (the 5 % are the probabilities' other rounding, drawn
+    anew by each chunk's own maximum)."""
+
+    generator = torch.Generator(device=gpu_device).manual_seed(context)
+    pool, (hq, hkv) = context + 100, heads
+    key, value = (torch.randn(pool, hkv, dim, device=gpu_device, generator=generator).to(dtype) for _ in range(2))
+    slots = torch.randperm(pool, device=gpu_device, generator=generator)[:context]
+    slots[context // 3] = -1  # an invisible key
+    table = _rows(context, spans, rows)
+    plan_spans = [(slots, int(s), int(s + n)) for _, s, n, _ in table.tolist()]
+    common = dict(num_q_heads=hq, num_kv_heads=hkv, head_dim=dim)
+    short = RepairAttentionPlan(plan_spans, **common)
+    assert short.info["split_tokens"] < 512 and short.info["num_combine"] > 0
+    whole = RepairAttentionPlan(plan_spans, split_tokens=8192, **common)
+    free = RepairAttentionPlan(plan_spans, allocation_free=True, **common)
+    query = (1.5 * torch.randn(short.num_queries, hq, dim, device=gpu_device, generator=generator)).to(dtype)
+    positions = torch.cat([torch.arange(s, e, device=gpu_device) for _, s, e in plan_spans])
+    hidden = torch.arange(context, device=gpu_device)[None] > positions[:, None]
+    hidden[:, context // 3] = True
+    safe = slots.clamp(min=0)
+    errors = []
+    for plan in (short, whole, free):
+        got = plan.run(query, key, value).double()
+        total = 0.0
+        for head in range(hq):
+            k, v = key[safe, head // (hq // hkv)].double(), value[safe, head // (hq // hkv)].double()
+            scores = (query[:, head].double() @ k.t()) / dim ** 0.5
+            weights = torch.softmax(scores.masked_fill(hidden, float("-inf")), dim=-1)
+            want, size = weights @ v, weights @ v.abs()
+            error = (got[:, head] - want).abs()
+            assert (error <= 2.0 ** -8 * size + 2.0 ** -9 * want.abs() + 1e-5).all()
+            total += float((error ** 2).sum())
+        errors.append(total ** 0.5)
+    assert errors[0] <= 1.05 * errors[1] and errors[2] == errors[0], errors

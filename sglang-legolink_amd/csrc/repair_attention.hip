@@ -965,15 +965,28 @@ constexpr double kCombineLaunchTiles = 2.0;
 // 2,048 keys it takes 5 us for 4 chunks, 7 us for 16 (0.1-0.17 us each), and
 // 45 us for 512 of a single span over 32k keys.
 constexpr double kCombineChunkTiles = 0.05;
+// Wide partials (chunks below 512 keys) are small plans' whole memory traffic,
+// written and read back by few workgroups: 54 16-row spans over 2.5k keys
+// (16/2 heads) took 29.2 us with 32 MB of them and 27.9 us with 512-key chunks
+// and 12 MB of 16-bit ones, though their items were 3 of 11 tiles shorter.
+constexpr double kWidePartialBytesPerTile = 4.5e6;
+// In a plan that leaves compute units idle the combine's launch itself counts,
+// on the host too: a single query over 296 keys takes 10.8 us whole and 12.3 us
+// in five chunks.
+constexpr double kSmallCombineTiles = 1.5;
+constexpr double kWideTiles = 1.0;  // five 16-row spans over 3k keys (64/8 heads): 22.1 us at 320 keys, 21.3 at 512
 constexpr int64_t kRefillTiles = 2;  // an item's slot-list refill (every kDmaMaxRange keys): drain and restart
 // A plan whose cost provably exceeds `beat` returns early with a lower bound
 // of its cost (still above `beat`).
-// `workgroups` is a work item's workgroups, `partial_bytes` those of one partial
-// result (all query heads).  A plan whose partials need more than
-// `workspace_limit` bytes (0: no limit) costs HUGE_VAL.
+// `groups` also gives each group's workgroups per KV head (a window of more
+// pairs than one workgroup holds takes two); `partial_bytes` are those of one
+// 16-bit partial result (all query heads), `wide` says that they are wide,
+// `small` that 512-key chunks leave compute units idle.  A
+// plan whose partials need more than `workspace_limit` bytes (0: no limit)
+// costs HUGE_VAL.
 template <typename Groups>
-double plan_cost_estimate(int64_t split, int64_t workgroups, int64_t partial_bytes, int64_t workspace_limit,
-                          double beat, Groups &&groups) {
+double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t partial_bytes, bool wide, bool small,
+                          int64_t workspace_limit, double beat, Groups &&groups) {
   // A group of `needed` keys makes needed / split full chunks and one shorter
   // one.  Costs are whole numbers of tiles, so their sums are exact in double
   // and do not depend on the order they are added in.
@@ -984,34 +997,35 @@ double plan_cost_estimate(int64_t split, int64_t workgroups, int64_t partial_byt
   const double full_cost = static_cast<double>(tiles_of(split));
   int64_t partials = 0, count = 0, most_chunks = 0;
   double total = 0.0, longest = 0.0;
-  groups([&](int64_t needed, int64_t group_partials) {
+  groups([&](int64_t needed, int64_t group_partials, int64_t workgroups) {
     const int64_t full = needed / split, rest = needed - full * split;
-    count += full + (rest > 0);
+    count += workgroups * (full + (rest > 0));
     most_chunks = full + (rest > 0) > most_chunks ? full + (rest > 0) : most_chunks;
-    total += static_cast<double>(full) * full_cost;
+    total += static_cast<double>(workgroups * full) * full_cost;
     if (full > 0) longest = full_cost > longest ? full_cost : longest;
     if (rest > 0) {
       const double cost = static_cast<double>(tiles_of(rest));
-      total += cost;
+      total += static_cast<double>(workgroups) * cost;
       longest = cost > longest ? cost : longest;
     }
     partials += group_partials;
   });
   double combine_cost = 0.0;
-  const double bytes = static_cast<double>(partials) * static_cast<double>(partial_bytes);
+  const double bytes = static_cast<double>(partials) * static_cast<double>(wide ? 2 * partial_bytes : partial_bytes);
   if (workspace_limit > 0 && bytes > static_cast<double>(workspace_limit)) return HUGE_VAL;
   if (partials > 0)
-    combine_cost = kCombineLaunchTiles + kCombineChunkTiles * static_cast<double>(most_chunks) +
-                   bytes / kPartialBytesPerTile;
+    combine_cost = kCombineLaunchTiles + (small ? kSmallCombineTiles : 0.0) + (wide ? kWideTiles : 0.0) +
+                   kCombineChunkTiles * static_cast<double>(most_chunks) +
+                   bytes / (wide ? kWidePartialBytesPerTile : kPartialBytesPerTile);
   if (count == 0) return combine_cost;
-  if (count * workgroups > 8 * kComputeUnits) {
+  if (count * num_kv_heads > 8 * kComputeUnits) {
     // Many rounds: the last one's imbalance is small against the total; it
     // leaves about half of the longest item to run alone.
-    return total * workgroups / kComputeUnits + 0.5 * longest + combine_cost;
+    return total * num_kv_heads / kComputeUnits + 0.5 * longest + combine_cost;
   }
   // No schedule ends before its longest item or before the CUs have run
   // every item's work.
-  const double spread = total * static_cast<double>(workgroups) / kComputeUnits;
+  const double spread = total * static_cast<double>(num_kv_heads) / kComputeUnits;
   const double bound = (longest > spread ? longest : spread) + combine_cost;
   if (bound > beat) return bound;
   double makespan = 0.0;
@@ -1020,22 +1034,22 @@ double plan_cost_estimate(int64_t split, int64_t workgroups, int64_t partial_byt
   static_assert(kItemOverheadTiles == 3.0, "the schedule counts whole tiles");
   const int64_t max_cost = tiles_of(split);
   std::vector<int64_t> cost_count(static_cast<size_t>(max_cost + 1), 0);
-  groups([&](int64_t needed, int64_t) {
+  groups([&](int64_t needed, int64_t, int64_t workgroups) {
     const int64_t full = needed / split, rest = needed - full * split;
-    cost_count[static_cast<size_t>(max_cost)] += full;
-    if (rest > 0) ++cost_count[static_cast<size_t>(tiles_of(rest))];
+    cost_count[static_cast<size_t>(max_cost)] += workgroups * full;
+    if (rest > 0) cost_count[static_cast<size_t>(tiles_of(rest))] += workgroups;
   });
   std::vector<int64_t> item_cost;
   item_cost.reserve(static_cast<size_t>(count));
   for (int64_t c = max_cost; c > 0; --c) item_cost.insert(item_cost.end(), static_cast<size_t>(cost_count[c]), c);
   const int64_t n = static_cast<int64_t>(item_cost.size());
-  if (n * workgroups <= 2 * kComputeUnits) {
+  if (n * num_kv_heads <= 2 * kComputeUnits) {
     // At most two rounds: the workgroups beyond the first 256 start when the
     // first round has ended (measured on c2: its 4 extra workgroups started
     // 72 us into an 82 us kernel, not when the first short items freed their
     // CUs), so the rounds' longest items add up.
     int64_t second = 0;
-    for (int64_t g = kComputeUnits; g < n * workgroups; ++g) {
+    for (int64_t g = kComputeUnits; g < n * num_kv_heads; ++g) {
       const int64_t cost = item_cost[static_cast<size_t>(g % n)];  // grid order: items, then KV heads
       second = cost > second ? cost : second;
     }
@@ -1046,7 +1060,7 @@ double plan_cost_estimate(int64_t split, int64_t workgroups, int64_t partial_byt
     // counted by free time and the earliest is found by moving forward.
     std::vector<int32_t> free_from(1, kComputeUnits);
     int64_t now = 0, last_end = 0;
-    for (int64_t h = 0; h < workgroups; ++h) {
+    for (int64_t h = 0; h < num_kv_heads; ++h) {
       for (const int64_t cost : item_cost) {
         while (free_from[static_cast<size_t>(now)] == 0) ++now;
         --free_from[static_cast<size_t>(now)];
@@ -1336,7 +1350,8 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     window_keys[k] = needed;
   }
   const int64_t dim = head_dim > 0 ? head_dim : 128;
-  const int64_t workgroups = num_kv_heads * (kMaxPairs / max_pairs(static_cast<int>(dim)));
+  const int64_t workgroup_pairs = max_pairs(static_cast<int>(dim));
+  auto window_workgroups = [&](const Window &w) { return (w.pair_count + workgroup_pairs - 1) / workgroup_pairs; };
   const int64_t partial_bytes = num_q_heads * (kQueries * dim * 2 + 2 * kQueries * 4);  // of one partial slot
   int64_t split = split_tokens;
   if (split == 0) {
@@ -1349,10 +1364,20 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     // the maximum, then every multiple of the key tile within 256 of
     // the best: one tile more per item can save a round (c2: 2,112 keys make
     // 64 items, one round of 4 KV heads on 256 CUs, where 2,048 make 65).
+    // Lengths below 512 where 512-key chunks leave compute units idle: three
+    // 8-row spans over 2,048 keys (28/4 heads) take 24.2 us in 16 workgroups of
+    // 512 keys and 16.2 us in 52 of 128; where 512-key chunks fill the device,
+    // shorter ones only add rounds (15 spans over 32k keys: 108 us at 512, 122
+    // at 384, 234 at 128).
+    int64_t items_512 = 0;
+    for (size_t k = 0; k < windows.size(); ++k)
+      items_512 += window_workgroups(windows[k]) * ((window_keys[k] + 511) / 512);
+    const bool small = head_dim > 0 && items_512 * num_kv_heads < kComputeUnits;
     double best = -1.0;
     auto estimate = [&](int64_t candidate) {
       const double beat = best < 0.0 ? HUGE_VAL : best;
-      return plan_cost_estimate(candidate, workgroups, partial_bytes, workspace_limit, beat, [&](auto &&visit) {
+      return plan_cost_estimate(candidate, num_kv_heads, partial_bytes, head_dim > 0 && candidate < 512, small,
+                                workspace_limit, beat, [&](auto &&visit) {
         int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
         for (size_t k = 0; k < windows.size(); ++k) {
           const Window &w = windows[k];
@@ -1362,7 +1387,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
             partials += chunks > 1 ? chunks : 0;
           }
           next_tile = w.last > next_tile ? w.last : next_tile;
-          visit(window_keys[k], partials);
+          visit(window_keys[k], partials, window_workgroups(w));
         }
       });
     };
@@ -1373,15 +1398,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     int64_t longest = kTile;
     for (const int64_t keys : window_keys) longest = keys > longest ? keys : longest;
     longest = (longest + kTile - 1) / kTile * kTile;
-    // Lengths below 512 where 512-key chunks leave compute units idle: three
-    // 8-row spans over 2,048 keys (28/4 heads) take 24.2 us in 16 workgroups of
-    // 512 keys and 16.2 us in 52 of 128; where 512-key chunks fill the device,
-    // shorter ones only add rounds (15 spans over 32k keys: 108 us at 512, 122
-    // at 384, 234 at 128).
     std::vector<int64_t> candidates;
-    int64_t items_512 = 0;
-    for (const int64_t keys : window_keys) items_512 += (keys + 511) / 512;
-    const bool small = head_dim > 0 && items_512 * workgroups < kComputeUnits;
     if (small) candidates = {64, 128, 192, 256, 320, 384, 448};
     candidates.insert(candidates.end(), std::begin(kCoarse), std::end(kCoarse));
     for (int64_t c = kCoarse[16] * 3 / 2 / kTile * kTile; c < longest; c = c * 3 / 2 / kTile * kTile)

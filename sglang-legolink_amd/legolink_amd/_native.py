@@ -17,6 +17,8 @@ import os
 import threading
 from pathlib import Path
 
+import torch
+
 LIB_DIR = Path(__file__).resolve().parent / "lib"
 # LEGOLINK_KV_LIBRARY names another build of the library (the host-sanitized
 # one of the CPU sanitizer test).
@@ -440,6 +442,13 @@ def pointer_table(pointers: list[int]) -> ctypes.Array:
     for index, value in enumerate(pointers):
         table[index] = int(value)
     return table
+
+
+def stream_handle(stream, device) -> int:
+    """The hipStream_t of ``stream``, or of the current stream of ``device`` (a
+    tensor's device, so it has an index)."""
+
+    return stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def kv_link(args: LinkArgs, stream: int) -> None:

@@ -9,6 +9,7 @@ Flags that matter for parity:
 
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -31,6 +32,10 @@ CALIBRATION_OUTPUT = PACKAGE_DIR / "lib" / "liblegolink_calibration.so"
 # (host code only, built with the C compiler against this interpreter).
 HOST_SEQUENCES_SOURCE = PACKAGE_DIR.parent / "csrc" / "host_sequences.c"
 HOST_SEQUENCES_OUTPUT = PACKAGE_DIR / f"_host_sequences{sysconfig.get_config_var('EXT_SUFFIX')}"
+# The Python module that fills argument blocks from tensors (host code only,
+# built with the C++ compiler against this interpreter and its torch).
+LINK_ARGUMENTS_SOURCE = PACKAGE_DIR.parent / "csrc" / "link_arguments.cpp"
+LINK_ARGUMENTS_OUTPUT = PACKAGE_DIR / f"_link_arguments{sysconfig.get_config_var('EXT_SUFFIX')}"
 # The same library with its host code under AddressSanitizer and
 # UndefinedBehaviorSanitizer (device code unchanged), for the CPU tests of the
 # host entries; never loaded on a GPU.
@@ -68,8 +73,8 @@ def build_library(verbose: bool = False, *, sanitize_host: bool = False) -> Path
     """Compile every translation unit in parallel, then link the library; the
     output is replaced atomically.  ``sanitize_host`` builds the host-sanitized
     copy (SANITIZED_OUTPUT) instead.  The unsanitized build also builds the
-    calibration library (CALIBRATION_OUTPUT) and the host module
-    (HOST_SEQUENCES_OUTPUT)."""
+    calibration library (CALIBRATION_OUTPUT) and the host modules
+    (HOST_SEQUENCES_OUTPUT, LINK_ARGUMENTS_OUTPUT)."""
 
     output = SANITIZED_OUTPUT if sanitize_host else OUTPUT
     extra = SANITIZE_FLAGS if sanitize_host else []
@@ -96,6 +101,17 @@ def build_library(verbose: bool = False, *, sanitize_host: bool = False) -> Path
                                            str(HOST_SEQUENCES_SOURCE)],
                                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True),
                          HOST_SEQUENCES_SOURCE))
+            link_arguments_tmp = Path(scratch) / LINK_ARGUMENTS_OUTPUT.name
+            torch_dir = Path(importlib.util.find_spec("torch").origin).parent
+            jobs.append((subprocess.Popen([os.environ.get("CXX") or shutil.which("g++") or "c++", "-O2", "-std=c++17",
+                                           "-shared", "-fPIC", "-Wall", f"-I{INCLUDE_DIR}",
+                                           f"-I{torch_dir / 'include'}",
+                                           f"-I{torch_dir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+                                           f"-I{sysconfig.get_paths()['include']}", "-o", str(link_arguments_tmp),
+                                           str(LINK_ARGUMENTS_SOURCE), f"-L{torch_dir / 'lib'}", "-ltorch_python",
+                                           "-ltorch", "-ltorch_cpu", "-lc10"],
+                                          stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True),
+                         LINK_ARGUMENTS_SOURCE))
         failures = []
         for job, source in jobs:
             printed, _ = job.communicate()
@@ -116,6 +132,7 @@ def build_library(verbose: bool = False, *, sanitize_host: bool = False) -> Path
         if calibration is not None:
             os.replace(calibration_tmp, CALIBRATION_OUTPUT)
             os.replace(host_sequences_tmp, HOST_SEQUENCES_OUTPUT)
+            os.replace(link_arguments_tmp, LINK_ARGUMENTS_OUTPUT)
     return output
 
 

@@ -26,6 +26,12 @@ import torch
 
 from . import _native
 
+try:
+    from . import _link_arguments
+except ImportError as error:
+    raise ImportError("legolink_amd._link_arguments is not built: run `python -m legolink_amd.build` "
+                      "(or __graft_entry__.build())") from error
+
 # Reason reported when the HIP library cannot be loaded; the reference reports
 # "triton_not_installed" in the same position (legolink_triton.py:174-175).
 NATIVE_UNAVAILABLE_REASON = "hip_kv_link_not_built"
@@ -427,6 +433,27 @@ def _link_args(
     args.cos_sin_stride_row = int(cos_sin_cache.stride(0))
     args.cos_sin_stride_col = int(cos_sin_cache.stride(1))
     args.rotary_dim = int(rotary_dim)
+    if source_tables:
+        args.source_key_layers = ctypes_address(source_tables[0])
+        args.source_value_layers = ctypes_address(source_tables[1])
+        args.source_num_slots = int(source_key_buffers[0].shape[0])
+    _set_link_options(args, prefix_token_count, is_neox_style, waves_per_block, layers_per_wave, kernel,
+                      layer_groups_per_block, rounding, delta_staging)
+    # The pointer tables must outlive the call.
+    return args, (key_table, value_table, *source_tables)
+
+
+def _set_link_options(
+    args: _native.LinkArgs,
+    prefix_token_count: int,
+    is_neox_style: bool,
+    waves_per_block: int,
+    layers_per_wave: int,
+    kernel: int,
+    layer_groups_per_block: int,
+    rounding: str,
+    delta_staging: str,
+) -> None:
     args.is_neox_style = 1 if is_neox_style else 0
     args.prefix_token_count = int(prefix_token_count)
     args.kernel = int(kernel)
@@ -439,12 +466,6 @@ def _link_args(
     args.delta_staging = DELTA_STAGINGS[delta_staging]
     if delta_staging == "workgroup":
         args.waves_per_block = 0  # the workgroup holds every layer group: the library sizes it
-    if source_tables:
-        args.source_key_layers = ctypes_address(source_tables[0])
-        args.source_value_layers = ctypes_address(source_tables[1])
-        args.source_num_slots = int(source_key_buffers[0].shape[0])
-    # The pointer tables must outlive the call.
-    return args, (key_table, value_table, *source_tables)
 
 
 def ctypes_address(array: Any) -> int:
@@ -513,21 +534,30 @@ class PreparedKVLink:
         source_value_buffers = list(source_value_buffers or ())
         if not key_buffers or len(key_buffers) != len(value_buffers):
             raise ValueError("key_buffers and value_buffers must be equal-length, non-empty")
-        eligibility = _eligibility(
-            key_buffers,
-            value_buffers,
-            source_slots,
-            destination_slots,
-            local_positions,
-            global_positions,
-            cos_sin_cache,
-            rotary_dim,
-            repair_mask,
-            source_key_buffers,
-            source_value_buffers,
-        )
-        if not eligibility.supported:
-            _raise_unavailable(eligibility.reason)
+        # One native call checks every tensor and fills the block; the Python
+        # checks run where it declines, and name the reason.
+        args = _native.LinkArgs()
+        tables = (ctypes.c_void_p * ((4 if source_key_buffers else 2) * len(key_buffers)))()
+        filled = _native.library_available() and _link_arguments.fill_link(
+            ctypes.addressof(args), ctypes.addressof(tables), key_buffers, value_buffers, source_key_buffers,
+            source_value_buffers, source_slots, destination_slots, local_positions, global_positions,
+            cos_sin_cache, repair_mask, int(rotary_dim))
+        if not filled:
+            eligibility = _eligibility(
+                key_buffers,
+                value_buffers,
+                source_slots,
+                destination_slots,
+                local_positions,
+                global_positions,
+                cos_sin_cache,
+                rotary_dim,
+                repair_mask,
+                source_key_buffers,
+                source_value_buffers,
+            )
+            if not eligibility.supported:
+                _raise_unavailable(eligibility.reason)
         if not 0 <= int(prefix_token_count) <= int(source_slots.numel()):
             raise ValueError("prefix_token_count is outside the linked token range")
         key_buffer, value_buffer = key_buffers[0], value_buffers[0]
@@ -557,27 +587,33 @@ class PreparedKVLink:
             )
         if repair_mask is not None and repair_mask.dtype == torch.bool:
             repair_mask = repair_mask.view(torch.uint8)
-        self._args, self._tables = _link_args(
-            key_buffers,
-            value_buffers,
-            source_slots,
-            destination_slots,
-            local_positions,
-            global_positions,
-            cos_sin_cache,
-            prefix_token_count,
-            rotary_dim,
-            is_neox_style,
-            repair_mask,
-            self.launch_config.num_warps,
-            layers_per_wave,
-            kernel,
-            layer_groups_per_block,
-            source_key_buffers,
-            source_value_buffers,
-            rounding,
-            delta_staging,
-        )
+        if filled:
+            _set_link_options(args, prefix_token_count, is_neox_style, self.launch_config.num_warps,
+                              layers_per_wave, kernel, layer_groups_per_block, rounding, delta_staging)
+            # The pointer tables must outlive the calls.
+            self._args, self._tables = args, (tables,)
+        else:
+            self._args, self._tables = _link_args(
+                key_buffers,
+                value_buffers,
+                source_slots,
+                destination_slots,
+                local_positions,
+                global_positions,
+                cos_sin_cache,
+                prefix_token_count,
+                rotary_dim,
+                is_neox_style,
+                repair_mask,
+                self.launch_config.num_warps,
+                layers_per_wave,
+                kernel,
+                layer_groups_per_block,
+                source_key_buffers,
+                source_value_buffers,
+                rounding,
+                delta_staging,
+            )
         self.rounding = rounding
         if skipped_rows is not None:
             if (skipped_rows.dtype != torch.int64 or skipped_rows.numel() != 1
@@ -600,12 +636,17 @@ class PreparedKVLink:
         )
         self.device = key_buffer.device
         try:
-            info = _native.kv_link_describe(self._args)
+            self._launch_info = _native.kv_link_describe(self._args)
         except _native.NativeCallError as error:
             self._raise_for(error)
-        self.launch = _launch_record(info)
         self._lib = _native.load_library()
         self._args_ref = ctypes.byref(self._args)
+
+    @property
+    def launch(self) -> dict[str, Any]:
+        """Kernel and launch shape of the link."""
+
+        return _launch_record(self._launch_info)
 
     @staticmethod
     def _raise_for(error: _native.NativeCallError) -> None:
@@ -618,9 +659,7 @@ class PreparedKVLink:
         _raise_unavailable(error.reason)
 
     def __call__(self, stream: torch.cuda.Stream | None = None) -> None:
-        if stream is None:
-            stream = torch.cuda.current_stream(self.device)
-        status = self._lib.ll_kv_link(self._args_ref, ctypes.c_void_p(stream.cuda_stream))
+        status = self._lib.ll_kv_link(self._args_ref, ctypes.c_void_p(_native.stream_handle(stream, self.device)))
         if status != _native.LL_OK:
             self._raise_for(
                 _native.NativeCallError(
@@ -724,7 +763,7 @@ def fused_kv_link_inplace(
     and ValueError for a bad prefix or launch configuration, like the reference.
     """
 
-    fused_kv_link_layers_inplace(
+    PreparedKVLink(
         key_buffers=[key_buffer],
         value_buffers=[value_buffer],
         source_slots=source_slots,
@@ -739,7 +778,7 @@ def fused_kv_link_inplace(
         block_size=block_size,
         num_warps=num_warps,
         num_stages=num_stages,
-    )
+    )()
 
 
 def describe_link_launch(
@@ -831,57 +870,62 @@ class PreparedKVScatter:
         if not _native.library_available():
             _raise_unavailable(NATIVE_UNAVAILABLE_REASON)
         tensors = (*key_buffers, *value_buffers, destination_slots, repaired_keys, repaired_values)
-        if not all(tensor.is_cuda and tensor.device == key_buffer.device for tensor in tensors):
-            _raise_unavailable("cuda_tensors_required")
-        for key, value in zip(key_buffers, value_buffers, strict=True):
-            if key.ndim != 3 or value.ndim != 3:
-                _raise_unavailable("mha_3d_kv_buffers_required")
-            if key.shape != key_buffer.shape or value.shape != value_buffer.shape or (
-                key.shape[:2] != value.shape[:2]
-            ):
-                _raise_unavailable("kv_head_layout_mismatch")
-            if key.dtype != key_buffer.dtype or value.dtype != key_buffer.dtype:
-                _raise_unavailable("kv_dtype_mismatch")
-            if not key.is_contiguous() or not value.is_contiguous():
-                _raise_unavailable("contiguous_kv_buffers_required")
-        if key_buffer.dtype not in _KV_DTYPES:
-            _raise_unavailable("fp16_or_bf16_required")
-        if destination_slots.dtype not in _INDEX_DTYPES or not destination_slots.is_contiguous():
-            _raise_unavailable("integer_token_maps_required")
-        expected_k = (layers, rows, int(key_buffer.shape[1]), int(key_buffer.shape[2]))
-        expected_v = (layers, rows, int(value_buffer.shape[1]), int(value_buffer.shape[2]))
-        if tuple(repaired_keys.shape) != expected_k or tuple(repaired_values.shape) != expected_v:
-            raise ValueError(
-                f"repaired rows must be {expected_k} / {expected_v}, got "
-                f"{tuple(repaired_keys.shape)} / {tuple(repaired_values.shape)}"
-            )
-        if repaired_keys.dtype != key_buffer.dtype or repaired_values.dtype != key_buffer.dtype:
-            _raise_unavailable("kv_dtype_mismatch")
-        if not repaired_keys[0].is_contiguous() or not repaired_values[0].is_contiguous():
-            raise ValueError("repaired rows of each layer must be dense")
-        self.rows = rows
-        self.device = key_buffer.device
-        self._tables = (
-            _native.pointer_table([buffer.data_ptr() for buffer in key_buffers]),
-            _native.pointer_table([buffer.data_ptr() for buffer in value_buffers]),
-        )
+        # As in PreparedKVLink: one native call, or the Python checks.
         args = _native.ScatterArgs()
         args.struct_size = ctypes.sizeof(_native.ScatterArgs)
-        args.num_layers = layers
-        args.key_layers = ctypes_address(self._tables[0])
-        args.value_layers = ctypes_address(self._tables[1])
-        args.num_slots = int(key_buffer.shape[0])
-        args.num_heads = int(key_buffer.shape[1])
-        args.key_head_dim = int(key_buffer.shape[2])
-        args.value_head_dim = int(value_buffer.shape[2])
-        args.kv_dtype = _KV_DTYPES[key_buffer.dtype]
-        args.num_rows = rows
-        args.destination_slots = destination_slots.data_ptr()
-        args.destination_slots_dtype = _INDEX_DTYPES[destination_slots.dtype]
-        args.repaired_key = repaired_keys.data_ptr()
-        args.repaired_key_layer_stride = int(repaired_keys.stride(0)) if layers > 1 else 0
-        args.repaired_value = repaired_values.data_ptr()
-        args.repaired_value_layer_stride = int(repaired_values.stride(0)) if layers > 1 else 0
+        tables = (ctypes.c_void_p * (2 * layers))()
+        self._tables = (tables,)
+        if not _link_arguments.fill_scatter(ctypes.addressof(args), ctypes.addressof(tables), key_buffers,
+                                            value_buffers, destination_slots, repaired_keys, repaired_values):
+            if not all(tensor.is_cuda and tensor.device == key_buffer.device for tensor in tensors):
+                _raise_unavailable("cuda_tensors_required")
+            for key, value in zip(key_buffers, value_buffers, strict=True):
+                if key.ndim != 3 or value.ndim != 3:
+                    _raise_unavailable("mha_3d_kv_buffers_required")
+                if key.shape != key_buffer.shape or value.shape != value_buffer.shape or (
+                    key.shape[:2] != value.shape[:2]
+                ):
+                    _raise_unavailable("kv_head_layout_mismatch")
+                if key.dtype != key_buffer.dtype or value.dtype != key_buffer.dtype:
+                    _raise_unavailable("kv_dtype_mismatch")
+                if not key.is_contiguous() or not value.is_contiguous():
+                    _raise_unavailable("contiguous_kv_buffers_required")
+            if key_buffer.dtype not in _KV_DTYPES:
+                _raise_unavailable("fp16_or_bf16_required")
+            if destination_slots.dtype not in _INDEX_DTYPES or not destination_slots.is_contiguous():
+                _raise_unavailable("integer_token_maps_required")
+            expected_k = (layers, rows, int(key_buffer.shape[1]), int(key_buffer.shape[2]))
+            expected_v = (layers, rows, int(value_buffer.shape[1]), int(value_buffer.shape[2]))
+            if tuple(repaired_keys.shape) != expected_k or tuple(repaired_values.shape) != expected_v:
+                raise ValueError(
+                    f"repaired rows must be {expected_k} / {expected_v}, got "
+                    f"{tuple(repaired_keys.shape)} / {tuple(repaired_values.shape)}"
+                )
+            if repaired_keys.dtype != key_buffer.dtype or repaired_values.dtype != key_buffer.dtype:
+                _raise_unavailable("kv_dtype_mismatch")
+            if not repaired_keys[0].is_contiguous() or not repaired_values[0].is_contiguous():
+                raise ValueError("repaired rows of each layer must be dense")
+            self._tables = (
+                _native.pointer_table([buffer.data_ptr() for buffer in key_buffers]),
+                _native.pointer_table([buffer.data_ptr() for buffer in value_buffers]),
+            )
+            args.num_layers = layers
+            args.key_layers = ctypes_address(self._tables[0])
+            args.value_layers = ctypes_address(self._tables[1])
+            args.num_slots = int(key_buffer.shape[0])
+            args.num_heads = int(key_buffer.shape[1])
+            args.key_head_dim = int(key_buffer.shape[2])
+            args.value_head_dim = int(value_buffer.shape[2])
+            args.kv_dtype = _KV_DTYPES[key_buffer.dtype]
+            args.num_rows = rows
+            args.destination_slots = destination_slots.data_ptr()
+            args.destination_slots_dtype = _INDEX_DTYPES[destination_slots.dtype]
+            args.repaired_key = repaired_keys.data_ptr()
+            args.repaired_key_layer_stride = int(repaired_keys.stride(0)) if layers > 1 else 0
+            args.repaired_value = repaired_values.data_ptr()
+            args.repaired_value_layer_stride = int(repaired_values.stride(0)) if layers > 1 else 0
+        self.rows = rows
+        self.device = key_buffer.device
         args.waves_per_block = int(num_warps)
         self._args = args
         self._args_ref = ctypes.byref(args)
@@ -891,9 +935,8 @@ class PreparedKVScatter:
     def __call__(self, stream: torch.cuda.Stream | None = None) -> None:
         if self.rows == 0:
             return
-        if stream is None:
-            stream = torch.cuda.current_stream(self.device)
-        status = self._lib.ll_kv_scatter_rows(self._args_ref, ctypes.c_void_p(stream.cuda_stream))
+        status = self._lib.ll_kv_scatter_rows(self._args_ref,
+                                              ctypes.c_void_p(_native.stream_handle(stream, self.device)))
         if status != _native.LL_OK:
             reason = self._lib.ll_status_reason(status).decode()
             detail = self._lib.ll_last_error().decode()

@@ -235,17 +235,15 @@ def build_device_maps(plan: SegmentPlan, destination_slots: torch.Tensor, *, com
         args.repair_mask[s] = masks[s].data_ptr() if masks[s] is not None else None
     args.repair_destination_slots = repair.data_ptr() if plan.repair_count else None
     args.repair_capacity = plan.repair_count
-    if stream is None:
-        stream = torch.cuda.current_stream(device)
     device_table = None
     if args.num_segments > DEVICE_TABLE_RUNS:
         # Many runs: one copy of the run table to the device and one launch,
         # where the kernel arguments would take a launch per 56 runs.  The
         # copy is ordered before the builder on its stream.
-        with torch.cuda.stream(stream):
+        with torch.cuda.stream(stream):  # (None: the current stream)
             device_table = torch.from_numpy(table).pin_memory().to(device, non_blocking=True)
         args.device_segments = device_table.data_ptr()
-    _native.kv_build_link_maps(args, stream.cuda_stream)
+    _native.kv_build_link_maps(args, _native.stream_handle(stream, device))
     return DeviceMaps(maps=maps, masks=masks, repair_destination_slots=repair, run_table=device_table)
 
 
@@ -277,9 +275,7 @@ def order_link_maps(maps: torch.Tensor, mask: Optional[torch.Tensor], *, key_row
     args.workspace = workspace.data_ptr()
     args.workspace_bytes = int(workspace.numel())
     args.key_row = int(key_row)
-    if stream is None:
-        stream = torch.cuda.current_stream(maps.device)
-    _native.order_link_maps(args, stream.cuda_stream)
+    _native.order_link_maps(args, _native.stream_handle(stream, maps.device))
     return out, out_mask
 
 

@@ -869,20 +869,21 @@ class KVLinkExecutor:
     # -- link ---------------------------------------------------------------
     def _layer_groups(self, layers: list[int], max_position: int,
                       device: torch.device) -> list[tuple[list[int], RotarySpec]]:
-        groups: list[tuple[list[int], RotarySpec]] = []
+        # Layers sharing a rotary embedding form one group, checked once.
+        by_spec: dict[int, tuple[list[int], RotarySpec]] = {}
         for layer in layers:
             rotary = self.rotary_by_layer.get(layer)
             if rotary is None:
                 raise LinkRuntimeError(f"Layer {layer} has no supported rotary embedding for PIC.")
+            group = by_spec.get(id(rotary))
+            if group is not None:
+                group[0].append(layer)
+                continue
             rotary.ensure_cos_sin_cache_length(max_position)
             if rotary.cos_sin_cache.device != device:
                 rotary.cos_sin_cache = rotary.cos_sin_cache.to(device)
-            for group_layers, group_rotary in groups:
-                if group_rotary is rotary:
-                    group_layers.append(layer)
-                    break
-            else:
-                groups.append(([layer], rotary))
+            by_spec[id(rotary)] = ([layer], rotary)
+        groups = list(by_spec.values())
         return groups
 
     def prepare_link(self, pool: Any, destination_slots: torch.Tensor, link_plan: Mapping[str, Any], *,

@@ -214,12 +214,11 @@ class RepairAttentionPlan:
         args.query_positions = self.positions.data_ptr()
         args.workspace = self.workspace.data_ptr() if self.workspace is not None else None
         args.workspace_items = self.info["workspace_items"]
-        if stream is None:
-            stream = torch.cuda.current_stream(query.device)
+        handle = _native.stream_handle(stream, query.device)
         if self.allocation_free:
-            _native.repair_attention_noalloc(args, stream.cuda_stream)
+            _native.repair_attention_noalloc(args, handle)
         else:
-            _native.repair_attention(args, stream.cuda_stream)
+            _native.repair_attention(args, handle)
         return output
 
 

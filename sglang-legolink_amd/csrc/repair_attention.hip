@@ -334,6 +334,7 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   constexpr int kKSteps = D / 16;                        // 16-dim steps of the score MFMAs
   constexpr int kDimBlocks = D / 32;                     // 32-dim blocks of O^T
   constexpr int kChunksPerRow = D / 8;                   // 16-byte chunks per row
+  static_assert(D != 256 || kLead == 1, "head dim 256 gathers one tile ahead");
   constexpr int kGathers = kChunksPerRow / (kM32Threads / kWave);  // per wave, per tile, of K and of V
   constexpr int kRowBytes = D * 2;
   constexpr int kStageBytes = kTile * kRowBytes;         // one K or V tile
@@ -425,14 +426,16 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   // together with the queries below, so that the gathers start two memory
   // round trips after the launch (item, then slots) instead of after the
   // header, the entries, the queries, the slot list and a barrier in a row.
-  // All loads of a group are unconditional (past the chunk's end its last key
-  // is read again and dropped) and keep the words as they come (an int32 slot
-  // has no high word), so that no wait and no branch separates them.
+  // The loads are unconditional (past the chunk's end its last key is read
+  // again and dropped) and keep the words as they come (an int32 slot has no
+  // high word), so that no wait separates them; short chunks skip the last
+  // three quarters of the list's by one scalar branch.
   constexpr int kFill = D == 256 ? 4 : 8;  // (registers)
   unsigned lead_lo[kLead][kGathers], lead_hi[kLead][kGathers], list_lo[kFill], list_hi[kFill];
   auto load_slots = [&](int chunk_begin, int first, bool lead) __attribute__((always_inline)) {
     const int last = min(load_stop - chunk_begin, kDmaMaxRange) - 1;
     const long long base = static_cast<long long>(kv_off) + chunk_begin;
+    const int first_wave = __builtin_amdgcn_readfirstlane(first);  // the wave's lowest entry
     auto load = [&](auto read) __attribute__((always_inline)) {
       if (lead) {
 #pragma unroll
@@ -442,8 +445,13 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
             read(min(t * kTile + g_token[j], last), lead_lo[t][j], lead_hi[t][j]);
       }
 #pragma unroll
-      for (int u = 0; u < kFill; ++u)
+      for (int u = 0; u < kFill / 4; ++u)
         read(min(first + u * kM32Threads, last), list_lo[u], list_hi[u]);
+      if (first_wave + kFill / 4 * kM32Threads <= last) {
+#pragma unroll
+        for (int u = kFill / 4; u < kFill; ++u)
+          read(min(first + u * kM32Threads, last), list_lo[u], list_hi[u]);
+      }
     };
     if (p.slots64) {
       const u32x2 *slots = static_cast<const u32x2 *>(p.slots) + base;
@@ -460,8 +468,12 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
       });
     }
   };
+  // Head dim 256 takes its one lead tile's slots from the list instead: eight
+  // loads more per lane cost more than the barrier (300 keys: 19.7 against
+  // 19.2 us).
+  constexpr bool kLeadFromList = D == 256;
   auto load_first_slots = [&](int chunk_begin) __attribute__((always_inline)) {
-    load_slots(chunk_begin, tid, true);
+    load_slots(chunk_begin, tid, !kLeadFromList);
   };
   if (load_stop <= kv_begin) load_stop = kv_begin;  // no keys: no slots, no tiles
   else
@@ -622,13 +634,15 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   // the tile loop may be left in flight.
   __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
   store_slots(tid);
+  if constexpr (!kLeadFromList) {
 #pragma unroll
-  for (int t = 0; t < kLead; ++t) {
-    int slots[kGathers];
+    for (int t = 0; t < kLead; ++t) {
+      int slots[kGathers];
 #pragma unroll
-    for (int j = 0; j < kGathers; ++j)
-      slots[j] = list_entry(lead_lo[t][j], slot_valid(lead_lo[t][j], lead_hi[t][j], t * kTile + g_token[j] < range));
-    if (t < tiles) gather_from(slots, k_ring + t * kStageBytes, v_ring + t * kStageBytes);
+      for (int j = 0; j < kGathers; ++j)
+        slots[j] = list_entry(lead_lo[t][j], slot_valid(lead_lo[t][j], lead_hi[t][j], t * kTile + g_token[j] < range));
+      if (t < tiles) gather_from(slots, k_ring + t * kStageBytes, v_ring + t * kStageBytes);
+    }
   }
   for (int base = tid + kFill * kM32Threads; base < tiles * kTile; base += kFill * kM32Threads) {
     load_slots(chunk_begin, base, false);
@@ -636,6 +650,11 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot list is written (the gathers stay in flight)
   workgroup_barrier();
+  if constexpr (kLeadFromList) {
+    int slots[kGathers];
+    gather_slots(0, slots);
+    gather_from(slots, k_ring, v_ring);
+  }
   static_assert(kStages == 2 || kStages == 4, "the tile loop is unrolled over the ring's stages");
   // One tile; the ring stage (t % kStages) is a compile-time constant, so
   // that the stage offsets of the LDS reads are immediates.

@@ -1000,12 +1000,14 @@ constexpr int64_t kRefillTiles = 2;  // an item's slot-list refill (every kDmaMa
 // `groups` also gives each group's workgroups per KV head (a window of more
 // pairs than one workgroup holds takes two); `partial_bytes` are those of one
 // 16-bit partial result (all query heads), `wide` says that they are wide,
-// `small` that 512-key chunks leave compute units idle.  A
-// plan whose partials need more than `workspace_limit` bytes (0: no limit)
+// `small` that 512-key chunks leave compute units idle, `combine_scale` is the
+// combine's time in key tiles against head dim 128 (a key tile takes 1.3 us
+// there, 2.4 us at head dim 256 and 0.7 us at 64; the combine's time does not
+// depend on it).  A plan whose partials need more than `workspace_limit` bytes (0: no limit)
 // costs HUGE_VAL.
 template <typename Groups>
 double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t partial_bytes, bool wide, bool small,
-                          int64_t workspace_limit, double beat, Groups &&groups) {
+                          double combine_scale, int64_t workspace_limit, double beat, Groups &&groups) {
   // A group of `needed` keys makes needed / split full chunks and one shorter
   // one.  Costs are whole numbers of tiles, so their sums are exact in double
   // and do not depend on the order they are added in.
@@ -1036,6 +1038,7 @@ double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t partial_b
     combine_cost = kCombineLaunchTiles + (small ? kSmallCombineTiles : 0.0) + (wide ? kWideTiles : 0.0) +
                    kCombineChunkTiles * static_cast<double>(most_chunks) +
                    bytes / (wide ? kWidePartialBytesPerTile : kPartialBytesPerTile);
+  combine_cost *= combine_scale;
   if (count == 0) return combine_cost;
   if (count * num_kv_heads > 8 * kComputeUnits) {
     // Many rounds: the last one's imbalance is small against the total; it
@@ -1396,7 +1399,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     auto estimate = [&](int64_t candidate) {
       const double beat = best < 0.0 ? HUGE_VAL : best;
       return plan_cost_estimate(candidate, num_kv_heads, partial_bytes, head_dim > 0 && candidate < 512, small,
-                                workspace_limit, beat, [&](auto &&visit) {
+                                128.0 / static_cast<double>(dim), workspace_limit, beat, [&](auto &&visit) {
         int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
         for (size_t k = 0; k < windows.size(); ++k) {
           const Window &w = windows[k];

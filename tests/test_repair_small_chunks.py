@@ -24,7 +24,7 @@ def _slot_bytes(heads, dim):
 
 
 @pytest.mark.parametrize("context,spans,rows,heads,dim", [
-    (2048, 3, 8, (28, 4), 128), (1300, 1, 1, (8, 8), 64), (1000, 5, 16, (64, 8), 256), (1500, 2, 16, (32, 1), 128),
+    (2048, 3, 8, (28, 4), 128), (2000, 2, 16, (16, 2), 64), (1000, 5, 16, (64, 8), 256), (1500, 2, 16, (32, 1), 128),
 ])
 def test_short_chunks_fill_idle_compute_units_with_wide_partials(context, spans, rows, heads, dim):
     table = _rows(context, spans, rows)
@@ -93,7 +93,7 @@ def test_bad_head_dims_and_limits_are_refused():
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("context,spans,rows,heads,dim", [
-    (2048, 3, 8, (28, 4), 128), (913, 2, 17, (8, 8), 64), (1000, 5, 1, (12, 4), 256), (2500, 1, 33, (32, 1), 128),
+    (2048, 3, 8, (28, 4), 128), (2113, 2, 17, (8, 8), 64), (1000, 5, 1, (12, 4), 256), (2500, 1, 33, (32, 1), 128),
     (4100, 6, 16, (7, 1), 64), (1471, 4, 16, (64, 8), 256),
 ])
 def test_short_chunks_are_as_exact_as_whole_ranges(gpu_device, context, spans, rows, heads, dim, dtype):

@@ -1177,6 +1177,62 @@ __global__ void __launch_bounds__(256) order_scatter_kernel(const OrderParams p)
   }
 }
 
+// Exact order within the buckets: one wave per bucket (the entries that the
+// scatter left in [offsets[b - 1], offsets[b]) of the tail of `maps`) counts its
+// entries by slot, scans the counts across its lanes and writes every entry to
+// its place in `out`.  A bucket's slots must be at most 64, one per lane.
+//
+// A batched link wants its repeated source rows next to each other: buckets
+// alone leave them up to 64 slots apart, which costs c3's link 3 %, and
+// torch's argsort and the gather of its result take 12 launches.  24 requests
+// x 4,096 tokens: 72 us (argsort and gather) -> 32 us in all four launches, the
+// batch's link as a whole 1,691 -> 1,655 us.  Latency-bound: a few entries per
+// wave, 64 bytes read and written per entry.
+constexpr int kOrderExactSlots = kWave;
+constexpr int kOrderExactWaves = 4;
+
+__global__ void __launch_bounds__(kOrderExactWaves * kWave) order_within_buckets_kernel(const OrderParams p) {
+  __shared__ int place_lds[kOrderExactWaves][kOrderExactSlots];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  int *place = place_lds[wave];  // counts, then next places, of this wave's bucket
+  const int bucket = blockIdx.x * kOrderExactWaves + wave;
+  const long long tail = p.count - p.prefix;
+  // Both bounds in [0, tail]: only a workspace shared by overlapping calls
+  // leaves others.
+  const long long begin = bucket == 0 ? 0 : min(max(static_cast<long long>(p.offsets[bucket - 1]), 0ll), tail);
+  const long long end = min(max(static_cast<long long>(p.offsets[bucket]), begin), tail);
+  place[lane] = 0;
+  __syncthreads();
+  const int slot_mask = (1 << p.shift) - 1;
+  const long long *key = p.key + p.prefix;
+  for (long long i = begin + lane; i < end; i += kWave)
+    atomicAdd(&place[static_cast<int>(key[i]) & slot_mask], 1);
+  __syncthreads();
+  const int own = place[lane];
+  int inclusive = own;
+#pragma unroll
+  for (int step = 1; step < kWave; step <<= 1) {
+    const int up = __shfl_up(inclusive, step, kWave);
+    if (lane >= step) inclusive += up;
+  }
+  __syncthreads();
+  place[lane] = inclusive - own;
+  __syncthreads();
+  for (long long i = begin + lane; i < end; i += kWave) {
+    const long long o = p.prefix + begin + atomicAdd(&place[static_cast<int>(key[i]) & slot_mask], 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p.out[r * p.cap + o] = p.maps[r * p.cap + p.prefix + i];
+    if (p.mask != nullptr) p.out_mask[o] = p.mask[p.prefix + i];
+  }
+  // The identity prefix stays in place.
+  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < p.prefix;
+       i += static_cast<long long>(gridDim.x) * blockDim.x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p.out[r * p.cap + i] = p.maps[r * p.cap + i];
+    if (p.mask != nullptr) p.out_mask[i] = p.mask[i];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
@@ -2203,7 +2259,8 @@ int ll_kv_build_link_maps(const ll_link_maps_args *a, ll_stream_t stream) {
 
 int64_t ll_order_maps_args_size(void) { return static_cast<int64_t>(sizeof(ll_order_maps_args)); }
 
-int ll_order_link_maps(const ll_order_maps_args *a, ll_stream_t stream) {
+static int order_link_maps(const ll_order_maps_args *a, int64_t *scratch_maps, uint8_t *scratch_mask, bool exact,
+                           ll_stream_t stream) {
   if (a == nullptr) return fail(LL_ERR_INVALID_ARGUMENT, "args is NULL");
   if (a->struct_size != static_cast<int64_t>(sizeof(ll_order_maps_args)))
     return fail(LL_ERR_INVALID_ARGUMENT, "struct_size %lld != %zu",
@@ -2236,6 +2293,22 @@ int ll_order_link_maps(const ll_order_maps_args *a, ll_stream_t stream) {
       (reinterpret_cast<uintptr_t>(a->workspace) & 15u) != 0)
     return fail(LL_ERR_INVALID_ARGUMENT, "workspace must be a 16-byte aligned device array of at least %d bytes",
                 LL_ORDER_WORKSPACE_BYTES);
+  int shift = 0;
+  while (((a->num_slots - 1) >> shift) >= kOrderBuckets) ++shift;
+  if (exact) {
+    if ((1ll << shift) > kOrderExactSlots)
+      return fail(LL_ERR_INVALID_ARGUMENT, "an exact order takes at most %lld slots",
+                  static_cast<long long>(kOrderBuckets) * kOrderExactSlots);
+    const uintptr_t scratch = reinterpret_cast<uintptr_t>(scratch_maps);
+    if (scratch_maps == nullptr || (scratch & 7u) != 0 || (a->mask != nullptr && scratch_mask == nullptr))
+      return fail(LL_ERR_INVALID_ARGUMENT, "an exact order needs scratch maps (8-byte aligned), and a scratch mask "
+                  "with a mask");
+    if ((scratch < in_begin + bytes && in_begin < scratch + bytes) ||
+        (scratch < out_begin + bytes && out_begin < scratch + bytes))
+      return fail(LL_ERR_INVALID_ARGUMENT, "the scratch maps overlap maps or out_maps");
+  }
+  // One slot per bucket is an exact order already.
+  const bool refine = exact && shift > 0 && a->count > a->prefix;
   OrderParams p;
   p.maps = reinterpret_cast<const long long *>(a->maps);
   p.key = p.maps + a->key_row * a->capacity;
@@ -2244,10 +2317,9 @@ int ll_order_link_maps(const ll_order_maps_args *a, ll_stream_t stream) {
   p.count = a->count;
   p.prefix = a->prefix;
   p.num_slots = a->num_slots;
-  p.shift = 0;
-  while (((a->num_slots - 1) >> p.shift) >= kOrderBuckets) ++p.shift;
-  p.out = reinterpret_cast<long long *>(a->out_maps);
-  p.out_mask = a->out_mask;
+  p.shift = shift;
+  p.out = reinterpret_cast<long long *>(refine ? scratch_maps : a->out_maps);
+  p.out_mask = refine ? scratch_mask : a->out_mask;
   p.counts = static_cast<int *>(a->workspace);
   p.offsets = p.counts + kOrderBuckets;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -2263,9 +2335,28 @@ int ll_order_link_maps(const ll_order_maps_args *a, ll_stream_t stream) {
   }
   const int64_t blocks = (a->count + 255) / 256;
   order_scatter_kernel<<<dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s>>>(p);
-  const hipError_t err = hipGetLastError();
+  hipError_t err = hipGetLastError();
   if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
+  if (refine) {
+    p.maps = p.out;
+    p.key = p.maps + a->key_row * a->capacity;
+    p.mask = a->mask != nullptr ? p.out_mask : nullptr;
+    p.out = reinterpret_cast<long long *>(a->out_maps);
+    p.out_mask = a->out_mask;
+    order_within_buckets_kernel<<<dim3(kOrderBuckets / kOrderExactWaves), dim3(kOrderExactWaves * kWave), 0, s>>>(p);
+    err = hipGetLastError();
+    if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
+  }
   return LL_OK;
+}
+
+int ll_order_link_maps(const ll_order_maps_args *a, ll_stream_t stream) {
+  return order_link_maps(a, nullptr, nullptr, false, stream);
+}
+
+int ll_order_link_maps_exact(const ll_order_maps_args *a, int64_t *scratch_maps, uint8_t *scratch_mask,
+                             ll_stream_t stream) {
+  return order_link_maps(a, scratch_maps, scratch_mask, true, stream);
 }
 
 }  // extern "C"

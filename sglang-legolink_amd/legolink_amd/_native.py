@@ -65,6 +65,7 @@ EXPORTED_SYMBOLS = (
     "ll_kv_build_link_maps",
     "ll_link_maps_args_size",
     "ll_order_link_maps",
+    "ll_order_link_maps_exact",
     "ll_order_maps_args_size",
     "ll_repair_attention_plan",
     "ll_repair_attention_plan_dim",
@@ -226,6 +227,7 @@ class LinkMapsArgs(ctypes.Structure):
 
 # Visit order of a map set (ll_order_link_maps).
 ORDER_BUCKETS = 16384
+ORDER_EXACT_SLOTS = 1 << 20  # most slots of ll_order_link_maps_exact
 ORDER_WORKSPACE_BYTES = 8 * ORDER_BUCKETS + 256
 
 
@@ -382,6 +384,8 @@ def load_library() -> ctypes.CDLL:
         lib.ll_link_maps_args_size.restype = _i64
         lib.ll_order_link_maps.argtypes = [ctypes.POINTER(OrderMapsArgs), _ptr]
         lib.ll_order_link_maps.restype = ctypes.c_int
+        lib.ll_order_link_maps_exact.argtypes = [ctypes.POINTER(OrderMapsArgs), _ptr, _ptr, _ptr]
+        lib.ll_order_link_maps_exact.restype = ctypes.c_int
         lib.ll_order_maps_args_size.argtypes = []
         lib.ll_order_maps_args_size.restype = _i64
         lib.ll_repair_attention_plan.argtypes = [_ptr, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64,
@@ -471,6 +475,12 @@ def kv_build_link_maps(args: LinkMapsArgs, stream: int) -> None:
 def order_link_maps(args: OrderMapsArgs, stream: int) -> None:
     args.struct_size = ctypes.sizeof(OrderMapsArgs)
     _check(load_library().ll_order_link_maps(ctypes.byref(args), _ptr(int(stream))))
+
+
+def order_link_maps_exact(args: OrderMapsArgs, scratch_maps: int, scratch_mask: int | None, stream: int) -> None:
+    args.struct_size = ctypes.sizeof(OrderMapsArgs)
+    _check(load_library().ll_order_link_maps_exact(ctypes.byref(args), _ptr(scratch_maps), _ptr(scratch_mask),
+                                                   _ptr(int(stream))))
 
 
 def repair_attention_plan(rows, num_q_heads: int, num_kv_heads: int, split_tokens: int = 0, head_dim: int = 0,

@@ -248,15 +248,17 @@ def build_device_maps(plan: SegmentPlan, destination_slots: torch.Tensor, *, com
 
 
 def order_link_maps(maps: torch.Tensor, mask: Optional[torch.Tensor], *, key_row: int, prefix: int,
-                    num_slots: int, workspace: torch.Tensor,
-                    stream: torch.cuda.Stream | None = None) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
+                    num_slots: int, workspace: torch.Tensor, stream: torch.cuda.Stream | None = None,
+                    exact: bool = False) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
     """A map set's entries [prefix, n) ordered by the slots of map row
     ``key_row`` (0: source slots, 1: destination slots), in buckets of 2^shift
     slots (16,384 buckets over the ``num_slots`` rows of the pool those slots
     index; one slot per bucket up to 16,384 rows); entries [0, prefix) stay
     first and in place, and the mask follows its entries.  ``workspace`` is a
     zeroed uint8 device tensor of ``_native.ORDER_WORKSPACE_BYTES`` that calls
-    on one stream may share (``ll_order_link_maps``)."""
+    on one stream may share (``ll_order_link_maps``).  ``exact`` orders the
+    entries within the buckets too (``ll_order_link_maps_exact``; at most
+    ``_native.ORDER_EXACT_SLOTS`` slots)."""
 
     if key_row not in (0, 1):
         raise ValueError("key_row must be 0 (source slots) or 1 (destination slots)")
@@ -275,7 +277,20 @@ def order_link_maps(maps: torch.Tensor, mask: Optional[torch.Tensor], *, key_row
     args.workspace = workspace.data_ptr()
     args.workspace_bytes = int(workspace.numel())
     args.key_row = int(key_row)
-    _native.order_link_maps(args, _native.stream_handle(stream, maps.device))
+    if exact:
+        scratch = torch.empty_like(maps)
+        scratch_mask = None if mask is None else torch.empty_like(mask)
+        # The scratch is used by the launches enqueued here only.  On a stream
+        # other than the current one the allocator is told so.
+        if stream is not None:
+            scratch.record_stream(stream)
+            if scratch_mask is not None:
+                scratch_mask.record_stream(stream)
+        _native.order_link_maps_exact(args, scratch.data_ptr(),
+                                      None if scratch_mask is None else scratch_mask.data_ptr(),
+                                      _native.stream_handle(stream, maps.device))
+    else:
+        _native.order_link_maps(args, _native.stream_handle(stream, maps.device))
     return out, out_mask
 
 

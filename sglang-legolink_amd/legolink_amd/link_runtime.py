@@ -480,7 +480,8 @@ class PreparedLink:
         self.stream_source_rows = (maps.request_count == 1 and not self.order_by_source
                                    and token_count * len(layers) * row_bytes > MEMORY_SIDE_CACHE_BYTES)
         sort_row = {"source": 0, "destination": 1}.get(self.visit_order)
-        if sort_row == 1 and order_workspace is None:
+        # Batches keep their own: they may be prepared on several streams at once.
+        if sort_row == 0 or (sort_row == 1 and order_workspace is None):
             order_workspace = torch.zeros(_native.ORDER_WORKSPACE_BYTES, dtype=torch.uint8,
                                           device=key_buffers[0].device)
         # delta_staging "table": a layer-major value pass writes every token's
@@ -520,15 +521,19 @@ class PreparedLink:
                 # at the head, with the fused entries after them.
                 split = prefix + int(np.count_nonzero(eager_entries[prefix:] == 0))
                 pieces = [(0, split, "fused", prefix), (split, count, "eager", 0)]
-            if sort_row == 1 and eager_entries is None and count - prefix > 1:
+            # The rows that the ordered slots index.
+            order_slots = int((source_arena.get_key_buffer(layers[0]) if sort_row == 0 and source_arena is not None
+                               else key_buffers[0]).shape[0])
+            if (eager_entries is None and count - prefix > 1
+                    and (sort_row == 1 or (sort_row == 0 and 0 < order_slots <= _native.ORDER_EXACT_SLOTS))):
                 # Destination order by the library's bucketed counting sort
-                # (three launches, where torch's argsort takes about ten).
-                # Source order stays an exact sort: a batch's repeated source
-                # rows must be adjacent to hit in cache (bucketed, c3's link
-                # ran 2.7-3.6 % slower: 8.59-8.65 against 8.35-8.39 ms).
+                # (three launches, where torch's argsort takes about twelve).
+                # Source order is exact (one launch more): a batch's repeated
+                # source rows must be adjacent to hit in cache (bucketed, c3's
+                # link ran 2.7-3.6 % slower: 8.59-8.65 against 8.35-8.39 ms).
                 device_maps, mask = link_maps.order_link_maps(
-                    device_maps, mask.view(torch.uint8) if mask is not None else None, key_row=1,
-                    prefix=prefix, num_slots=int(key_buffers[0].shape[0]), workspace=order_workspace)
+                    device_maps, mask.view(torch.uint8) if mask is not None else None, key_row=sort_row,
+                    prefix=prefix, num_slots=order_slots, workspace=order_workspace, exact=sort_row == 0)
                 self._kernel_maps.append(device_maps)
             elif (sort_row is not None or eager_entries is not None) and count - prefix > 1:
                 tail = device_maps[:, prefix:]

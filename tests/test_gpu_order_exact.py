@@ -27,6 +27,33 @@ CASES = [
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("with_mask", [False, True])
+@pytest.mark.parametrize("num_slots", [1, 16384, 70000, 1 << 22])
+@pytest.mark.parametrize("n,prefix", [(1, 0), (63, 0), (1025, 1), (2047, 64), (2048, 2048), (2048, 0), (2049, 0)])
+def test_small_maps_order_in_one_workgroup_as_in_three_launches(gpu_device, n, prefix, num_slots, with_mask):
+    """Sizes on both sides of the one-workgroup line: bucket order, the prefix and the masks kept."""
+
+    rng = np.random.default_rng([n, num_slots])
+    host = np.stack([rng.integers(0, 1 << 40, n), rng.integers(-2, num_slots + 2, n), rng.integers(0, 99, n),
+                     np.arange(n) * 5 + 1]).astype(np.int64)
+    mask_host = rng.integers(0, 2, n).astype(np.uint8)
+    mask = torch.from_numpy(mask_host).to(gpu_device) if with_mask else None
+    workspace = torch.zeros(_native.ORDER_WORKSPACE_BYTES, dtype=torch.uint8, device=gpu_device)
+    out, out_mask = link_maps.order_link_maps(torch.from_numpy(host).to(gpu_device), mask, key_row=1, prefix=prefix,
+                                              num_slots=num_slots, workspace=workspace)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:, :prefix], host[:, :prefix])
+    assert np.array_equal(got[:, np.argsort(got[3])], host)
+    shift = max(0, int(num_slots - 1).bit_length() - 14)
+    buckets = np.clip(got[1, prefix:], 0, num_slots - 1) >> shift
+    buckets[got[1, prefix:] >= num_slots] = _native.ORDER_BUCKETS - 1
+    assert (np.diff(buckets) >= 0).all()
+    if with_mask:
+        assert np.array_equal(out_mask.cpu().numpy()[np.argsort(got[3])], mask_host)
+    assert int(workspace.count_nonzero()) == 0 or n > 2048
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("key_row", [0, 1])
 @pytest.mark.parametrize("with_mask", [False, True])
 @pytest.mark.parametrize("case", CASES, ids=str)

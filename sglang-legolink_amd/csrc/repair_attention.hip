@@ -164,7 +164,8 @@ __host__ __device__ constexpr int partial_floats() { return kQueries * D / 2 + 2
 // in the space of two partial slots (16 D + 64 floats per head).  Plans with
 // chunks below 512 keys use them: such a chunk may split what one workgroup
 // would otherwise keep in fp32 from end to end, and the few partials of so
-// small a plan cost nothing (2,048 keys: 17.3 us either way).
+// small a plan cost little (three spans over 2,048 keys 17.3 -> 17.9 us, 16.3 us
+// since the combine takes them in groups).
 template <int D>
 __device__ inline float *partial_block(const AttnParams &p, int partial, int h, bool wide) {
   return p.ws + (static_cast<long long>(partial) * p.hq + (wide ? 2 * h : h)) * partial_floats<D>();
@@ -351,7 +352,7 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   // trip away instead of three in a row.  With the slots and queries requested
   // together below, the time before the first tile is that of its ~850
   // instructions, no longer of a chain of loads: 15 spans over 32k keys (28/4
-  // heads) 75.1 -> 73.2 us, 168 spans of 24 requests 153.7 -> 152.1 us.
+  // heads) 74.5 -> 72.5 us, 168 spans of 24 requests 153.9 -> 153.2 us.
   static_assert(kItemInts > kWave && kItemInts <= 2 * kWave, "two fields per lane");
   // The kernel arguments in one group of scalar loads, ahead of their uses.
   asm volatile("" ::"s"(p.items), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.slots), "s"(p.positions), "s"(p.num_queries),
@@ -470,7 +471,7 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   };
   // Head dim 256 takes its one lead tile's slots from the list instead: eight
   // loads more per lane cost more than the barrier (300 keys: 19.7 against
-  // 19.2 us).
+  // 19.5 us).
   constexpr bool kLeadFromList = D == 256;
   auto load_first_slots = [&](int chunk_begin) __attribute__((always_inline)) {
     load_slots(chunk_begin, tid, !kLeadFromList);
@@ -1042,14 +1043,15 @@ constexpr int64_t kRefillTiles = 2;  // an item's slot-list refill (every kDmaMa
 // `groups` also gives each group's workgroups per KV head (a window of more
 // pairs than one workgroup holds takes two); `partial_bytes` are those of one
 // 16-bit partial result (all query heads), `wide` says that they are wide,
-// `small` that 512-key chunks leave compute units idle, `combine_scale` is the
+// `small` that 512-key chunks leave compute units idle, `chunk_tiles` is the
+// combine's cost per chunk of the most split tile, `combine_scale` the
 // combine's time in key tiles against head dim 128 (a key tile takes 1.3 us
 // there, 2.4 us at head dim 256 and 0.7 us at 64; the combine's time does not
 // depend on it).  A plan whose partials need more than `workspace_limit` bytes (0: no limit)
 // costs HUGE_VAL.
 template <typename Groups>
 double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t partial_bytes, bool wide, bool small,
-                          double combine_scale, int64_t workspace_limit, double beat, Groups &&groups) {
+                          double chunk_tiles, double combine_scale, int64_t workspace_limit, double beat, Groups &&groups) {
   // A group of `needed` keys makes needed / split full chunks and one shorter
   // one.  Costs are whole numbers of tiles, so their sums are exact in double
   // and do not depend on the order they are added in.
@@ -1078,7 +1080,7 @@ double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t partial_b
   if (workspace_limit > 0 && bytes > static_cast<double>(workspace_limit)) return HUGE_VAL;
   if (partials > 0)
     combine_cost = kCombineLaunchTiles + (small ? kSmallCombineTiles : 0.0) + (wide ? kWideTiles : 0.0) +
-                   kCombineChunkTiles * static_cast<double>(most_chunks) +
+                   chunk_tiles * static_cast<double>(most_chunks) +
                    bytes / (wide ? kWidePartialBytesPerTile : kPartialBytesPerTile);
   combine_cost *= combine_scale;
   if (count == 0) return combine_cost;
@@ -1450,7 +1452,8 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     auto estimate = [&](int64_t candidate) {
       const double beat = best < 0.0 ? HUGE_VAL : best;
       return plan_cost_estimate(candidate, num_kv_heads, partial_bytes, head_dim > 0 && candidate < 512, small,
-                                128.0 / static_cast<double>(dim), workspace_limit, beat, [&](auto &&visit) {
+                                head_dim > 0 ? kCombineChunkTiles : 0.0, 128.0 / static_cast<double>(dim),
+                                workspace_limit, beat, [&](auto &&visit) {
         int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
         for (size_t k = 0; k < windows.size(); ++k) {
           const Window &w = windows[k];

@@ -511,7 +511,7 @@ typedef struct ll_repair_row {
 typedef struct ll_repair_attention_plan_info {
   int64_t num_items;               /* int32 [num_items, 86] work items (ABI 13) */
   int64_t num_combine;             /* int32 [num_combine, 4] combine items */
-  int64_t workspace_items;         /* partial results (see ll_repair_attention_args.workspace) */
+  int64_t workspace_items;         /* blocks of partial results per head (see ll_repair_attention_args.workspace) */
   int64_t split_tokens;            /* KV tokens per work item (the plan's choice when 0 was asked) */
   int64_t num_queries;             /* entries of the positions table: max(query_index + query_count) */
 } ll_repair_attention_plan_info;
@@ -538,9 +538,14 @@ typedef struct ll_repair_attention_args {
   int64_t num_combine;
   const int32_t *query_positions;  /* device copy of the plan's positions table [num_queries] */
   float *workspace;                /* device, 16-byte aligned: workspace_items x num_q_heads blocks of
-                                      8 * head_dim + 32 floats (16 queries' outputs in the KV dtype,
-                                      then 16 fp32 (maximum, sum) pairs) (ABI 14) */
-  int64_t workspace_items;
+                                      8 * head_dim + 32 floats (ABI 14).  A partial takes one block per
+                                      head (16 queries' outputs in the KV dtype, then 16 fp32 (maximum,
+                                      sum) pairs), or, wide, two slots: of their 2 x num_q_heads blocks
+                                      head h takes 2 h and 2 h + 1 (16 queries' outputs in fp32, then
+                                      the pairs).  The plan's tables say which: bit 8 of an item's pair
+                                      count (int 5) and of a combine item's query count (int 1) is set
+                                      for wide partials */
+  int64_t workspace_items;         /* blocks per head: the plan's workspace_items */
 } ll_repair_attention_args;
 
 int ll_repair_attention_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_heads,
@@ -555,6 +560,14 @@ int ll_repair_attention_plan(const ll_repair_row *rows, int64_t num_rows, int64_
  * are tried where they fill idle compute units, and workspace_limit, the bytes
  * of partial results that the plan may need (0: any;
  * ll_repair_attention_noalloc takes LL_REPAIR_SCRATCH_BYTES).
+ *
+ * Where the chunks are shorter than 512 keys, or split a tile that
+ * ll_repair_attention_plan keeps whole, the partials are wide: fp32 outputs,
+ * two slots each (see ll_repair_attention_args.workspace), so that no tile's
+ * result is rounded in between that was not before.  A chunk length of 512 and
+ * more that the caller gives keeps 16-bit partials: size and fill the tables
+ * with the same split_tokens (the plan is kept between the two calls), not the
+ * filling call with the length that the sizing call chose.
  */
 int ll_repair_attention_plan_dim(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_heads,
                                  int64_t num_kv_heads, int64_t head_dim, int64_t split_tokens,

@@ -161,10 +161,12 @@ struct F16 {
 template <int D>
 __host__ __device__ constexpr int partial_floats() { return kQueries * D / 2 + 2 * kQueries; }
 // A wide partial keeps O / l in fp32, [16][D] floats and then (m, l) as above,
-// in the space of two partial slots (16 D + 64 floats per head).  Plans with
-// chunks below 512 keys use them: such a chunk may split what one workgroup
-// would otherwise keep in fp32 from end to end, and the few partials of so
-// small a plan cost little (three spans over 2,048 keys 17.3 -> 17.9 us, 16.3 us
+// in the space of two partial slots (16 D + 64 floats per head).  Plans that
+// split what one workgroup would otherwise keep in fp32 from end to end use
+// them: those with chunks below 512 keys, and those whose chunks split a tile
+// that the plan made without the head dim keeps whole (at head dim 256, whose
+// windows take two workgroups each).  The few partials of so small a plan cost
+// little (three spans over 2,048 keys 17.3 -> 17.9 us, 16.3 us
 // since the combine takes them in groups).
 template <int D>
 __device__ inline float *partial_block(const AttnParams &p, int partial, int h, bool wide) {
@@ -1321,6 +1323,7 @@ struct RepairPlan {
   std::vector<int32_t> items, combine, positions;
   std::vector<int32_t> sorted;  // reordering space for the items
   ll_repair_attention_plan_info info{};
+  bool as_given = false;  // the chosen chunk length, given, makes the same plan
 };
 
 // head_dim 0: not known (planned as 128, with chunks of at least 512 keys).
@@ -1428,7 +1431,11 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
   const int64_t workgroup_pairs = max_pairs(static_cast<int>(dim));
   auto window_workgroups = [&](const Window &w) { return (w.pair_count + workgroup_pairs - 1) / workgroup_pairs; };
   const int64_t partial_bytes = num_q_heads * (kQueries * dim * 2 + 2 * kQueries * 4);  // of one partial slot
+  const int64_t blind_partial_bytes = num_q_heads * (kQueries * 128 * 2 + 2 * kQueries * 4);
   int64_t split = split_tokens;
+  // Keys of the longest tile that the plan without the head dim keeps whole: a
+  // chosen length that splits such a tile takes wide partials.
+  int64_t whole_keys = 0;
   if (split == 0) {
     // Pick the chunk length whose plan finishes first on a model of the
     // device: one workgroup per CU at a time (its LDS allows no more),
@@ -1447,55 +1454,72 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     int64_t items_512 = 0;
     for (size_t k = 0; k < windows.size(); ++k)
       items_512 += window_workgroups(windows[k]) * ((window_keys[k] + 511) / 512);
-    const bool small = head_dim > 0 && items_512 * num_kv_heads < kComputeUnits;
-    double best = -1.0;
-    auto estimate = [&](int64_t candidate) {
-      const double beat = best < 0.0 ? HUGE_VAL : best;
-      return plan_cost_estimate(candidate, num_kv_heads, partial_bytes, head_dim > 0 && candidate < 512, small,
-                                head_dim > 0 ? kCombineChunkTiles : 0.0, 128.0 / static_cast<double>(dim),
-                                workspace_limit, beat, [&](auto &&visit) {
-        int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
-        for (size_t k = 0; k < windows.size(); ++k) {
-          const Window &w = windows[k];
-          int64_t partials = 0;
-          for (int64_t t = w.first > next_tile ? w.first : next_tile; t < w.last; ++t) {
-            const int64_t chunks = (tiles[t].needed + candidate - 1) / candidate;
-            partials += chunks > 1 ? chunks : 0;
-          }
-          next_tile = w.last > next_tile ? w.last : next_tile;
-          visit(window_keys[k], partials, window_workgroups(w));
-        }
-      });
-    };
-    // Beyond 7,680 keys the lengths grow by half up to the longest window's
-    // keys, which leaves every window whole (no partials, no combine).
-    static const int64_t kCoarse[] = {512,  640,  768,  1024, 1280, 1536, 1792, 2048, 2304,
-                                      2560, 3072, 3584, 4096, 4608, 5120, 6144, 7680};
+    const bool idle_units = head_dim > 0 && items_512 * num_kv_heads < kComputeUnits;
     int64_t longest = kTile;
     for (const int64_t keys : window_keys) longest = keys > longest ? keys : longest;
     longest = (longest + kTile - 1) / kTile * kTile;
-    std::vector<int64_t> candidates;
-    if (small) candidates = {64, 128, 192, 256, 320, 384, 448};
-    candidates.insert(candidates.end(), std::begin(kCoarse), std::end(kCoarse));
-    for (int64_t c = kCoarse[16] * 3 / 2 / kTile * kTile; c < longest; c = c * 3 / 2 / kTile * kTile)
-      candidates.push_back(c);
-    if (longest > kCoarse[16]) candidates.push_back(longest);
-    for (const int64_t candidate : candidates) {
-      const double cost = estimate(candidate);
-      if (best < 0.0 || cost <= best) {
-        best = cost;
-        split = candidate;
+    // The search, knowing the head dim or not.
+    auto choose = [&](bool dim_known) {
+      const bool small = dim_known && idle_units;
+      int64_t chosen = 0;
+      double best = -1.0;
+      auto estimate = [&](int64_t candidate) {
+        const double beat = best < 0.0 ? HUGE_VAL : best;
+        const bool wide = dim_known && (candidate < 512 || candidate < whole_keys);
+        return plan_cost_estimate(candidate, num_kv_heads, dim_known ? partial_bytes : blind_partial_bytes, wide, small,
+                                  dim_known ? kCombineChunkTiles : 0.0,
+                                  dim_known ? 128.0 / static_cast<double>(dim) : 1.0,
+                                  dim_known ? workspace_limit : 0, beat, [&](auto &&visit) {
+          int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
+          for (size_t k = 0; k < windows.size(); ++k) {
+            const Window &w = windows[k];
+            int64_t partials = 0;
+            for (int64_t t = w.first > next_tile ? w.first : next_tile; t < w.last; ++t) {
+              const int64_t chunks = (tiles[t].needed + candidate - 1) / candidate;
+              partials += chunks > 1 ? chunks : 0;
+            }
+            next_tile = w.last > next_tile ? w.last : next_tile;
+            visit(window_keys[k], partials, dim_known ? window_workgroups(w) : 1);
+          }
+        });
+      };
+      // Beyond 7,680 keys the lengths grow by half up to the longest window's
+      // keys, which leaves every window whole (no partials, no combine).
+      static const int64_t kCoarse[] = {512,  640,  768,  1024, 1280, 1536, 1792, 2048, 2304,
+                                        2560, 3072, 3584, 4096, 4608, 5120, 6144, 7680};
+      std::vector<int64_t> candidates;
+      if (small) candidates = {64, 128, 192, 256, 320, 384, 448};
+      candidates.insert(candidates.end(), std::begin(kCoarse), std::end(kCoarse));
+      for (int64_t c = kCoarse[16] * 3 / 2 / kTile * kTile; c < longest; c = c * 3 / 2 / kTile * kTile)
+        candidates.push_back(c);
+      if (longest > kCoarse[16]) candidates.push_back(longest);
+      for (const int64_t candidate : candidates) {
+        const double cost = estimate(candidate);
+        if (best < 0.0 || cost <= best) {
+          best = cost;
+          chosen = candidate;
+        }
       }
-    }
-    const int64_t coarse = split;
-    for (int64_t candidate = coarse - 256; candidate <= coarse + 256; candidate += kTile) {
-      if (candidate < (small ? kTile : 512) || candidate == coarse) continue;
-      const double cost = estimate(candidate);
-      if (cost < best || (cost == best && candidate > split)) {
-        best = cost;
-        split = candidate;
+      const int64_t coarse = chosen;
+      for (int64_t candidate = coarse - 256; candidate <= coarse + 256; candidate += kTile) {
+        if (candidate < (small ? kTile : 512) || candidate == coarse) continue;
+        const double cost = estimate(candidate);
+        if (cost < best || (cost == best && candidate > chosen)) {
+          best = cost;
+          chosen = candidate;
+        }
       }
+      return chosen;
+    };
+    // At head dim 128 a plan that fills the device differs from the blind one
+    // by a cost that only falls with the chunk length (the combine's, per chunk
+    // of the most split tile), so its chunks are never the shorter ones.
+    if (head_dim > 0 && (idle_units || head_dim != 128)) {
+      const int64_t blind = choose(false);
+      for (const Tile &tile : tiles)
+        if (tile.needed <= blind && tile.needed > whole_keys) whole_keys = tile.needed;
     }
+    split = choose(head_dim > 0);
   }
   // Each tile's key chunks, and the partial slots and combine item of a tile
   // with more than one.
@@ -1506,9 +1530,10 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     chunks[t] = (tiles[t].needed + split - 1) / split;
     n_partial += chunks[t] > 1 ? chunks[t] : 0;
   }
-  // Wide partials, which take two slots each, for chunks below 512 keys (where
-  // the workspace limit allows them).
-  const bool wide = head_dim > 0 && split < 512 && n_partial > 0 && n_partial <= kIntMax / 2 &&
+  // Wide partials, which take two slots each, for chunks below 512 keys or that
+  // split a tile which would otherwise stay whole (where the workspace limit
+  // allows them: a chosen length always fits it, a given one may not).
+  const bool wide = head_dim > 0 && (split < 512 || split < whole_keys) && n_partial > 0 && n_partial <= kIntMax / 2 &&
                     (workspace_limit == 0 ||
                      static_cast<double>(2 * n_partial) * static_cast<double>(partial_bytes) <=
                          static_cast<double>(workspace_limit));
@@ -1580,6 +1605,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
   out.info.workspace_items = n_partial;
   out.info.split_tokens = split;
   out.info.num_queries = num_queries;
+  out.as_given = !wide || split < 512;
   return LL_OK;
 }
 
@@ -1621,7 +1647,7 @@ int ll_repair_attention_plan_dim(const ll_repair_row *rows, int64_t num_rows, in
       static_cast<int64_t>(kept.rows.size()) == num_rows && kept.num_q_heads == num_q_heads &&
       kept.num_kv_heads == num_kv_heads && kept.head_dim == head_dim &&
       kept.workspace_limit == workspace_limit &&
-      (split_tokens == kept.split_in || split_tokens == kept.info.split_tokens) &&
+      (split_tokens == kept.split_in || (kept.as_given && split_tokens == kept.info.split_tokens)) &&
       (num_rows == 0 || memcmp(kept.rows.data(), rows, static_cast<size_t>(num_rows) * sizeof(ll_repair_row)) == 0);
   if (!same_rows) {
     kept.num_q_heads = -1;  // invalid until computed

@@ -502,11 +502,10 @@ def repair_attention_plan(rows, num_q_heads: int, num_kv_heads: int, split_token
     items = np.empty((info.num_items, REPAIR_ITEM_INTS), dtype=np.int32)
     combine = np.empty((info.num_combine, REPAIR_COMBINE_INTS), dtype=np.int32)
     positions = np.empty(info.num_queries, dtype=np.int32)
-    # The sizing call chose the chunk length: the filling call takes it as
-    # given instead of searching again (same plan, half the host time).
-    chosen = int(info.split_tokens)
+    # The same arguments: the filling call finds the plan that the sizing call
+    # made on this thread.
     _check(lib.ll_repair_attention_plan_dim(rows_ptr, rows.shape[0], int(num_q_heads), int(num_kv_heads),
-                                            int(head_dim), chosen, int(workspace_limit),
+                                            int(head_dim), int(split_tokens), int(workspace_limit),
                                             items.ctypes.data if items.size else None, info.num_items,
                                             combine.ctypes.data if combine.size else None, info.num_combine,
                                             positions.ctypes.data if positions.size else None, positions.size,

@@ -60,6 +60,59 @@ def test_head_dim_256_plans_one_round_of_its_two_workgroups_per_window(context, 
     assert info.num_items * 4 * 2 <= 256
 
 
+def _batch(requests, context, spans, rows):
+    """The rows of `requests` requests of `context` keys with `spans` spans each."""
+
+    one = _rows(context, spans, rows)
+    table = np.concatenate([one] * requests)
+    table[:, 0] = np.arange(len(table)) * rows
+    table[:, 3] = np.repeat(np.arange(requests) * context, spans)
+    return table
+
+
+def _check_splits_are_wide(table, heads, dim, limit=0):
+    """A tile that the plan made without the head dim keeps whole, in fp32 from
+    end to end, is whole here too, or its partials are fp32.  Returns whether
+    the plan splits such a tile."""
+
+    blind = _native.repair_attention_plan(table, *heads, 0)[1]
+    items, combine, _, info = _native.repair_attention_plan(table, *heads, 0, head_dim=dim, workspace_limit=limit)
+    newly_split = set(combine[:, 0].tolist()) - set(blind[:, 0].tolist())
+    if newly_split:
+        assert (combine[:, 1] & WIDE).all() and (items[:, 5] & WIDE).all(), (heads, dim, info.split_tokens)
+        assert info.workspace_items == 2 * int(combine[:, 3].sum())
+    assert limit == 0 or info.workspace_items * _slot_bytes(heads[0], dim) <= limit
+    return bool(newly_split)
+
+
+NEWLY_SPLIT = [(6, 938, 10, 32, (28, 4)), (12, 875, 4, 32, (32, 1)), (14, 1727, 2, 32, (64, 8))]
+
+
+@pytest.mark.parametrize("requests,context,spans,rows,heads", NEWLY_SPLIT)
+def test_ranges_that_stayed_whole_split_into_wide_partials(requests, context, spans, rows, heads):
+    table = _batch(requests, context, spans, rows)
+    for limit in (0, 64 << 20, 1 << 20):
+        _check_splits_are_wide(table, heads, 256, limit)
+    # A chunk length that the caller gives (512 keys and more) keeps its 16-bit
+    # partials, whatever was planned before on this thread.
+    chosen = _native.repair_attention_plan(table, *heads, 0, head_dim=256)
+    given = _native.repair_attention_plan(table, *heads, max(512, int(chosen[3].split_tokens)), head_dim=256)
+    assert not (given[1][:, 1] & WIDE).any()
+
+
+def test_drawn_plans_never_lose_the_partials_precision():
+    rng = np.random.default_rng(7)
+    split = 0
+    for _ in range(400):
+        dim = int(rng.choice([64, 128, 256, 256]))
+        heads = [(28, 4), (64, 8), (14, 2), (7, 1), (8, 8), (16, 2), (32, 1)][rng.integers(7)]
+        context = int(np.exp(rng.uniform(np.log(512), np.log(32768))))
+        rows = int(rng.choice([1, 8, 16, 32]))
+        spans = int(np.exp(rng.uniform(0, np.log(max(1, min(64, context // 33))))))
+        split += _check_splits_are_wide(_batch(int(rng.integers(1, 25)), context, spans, rows), heads, dim)
+    assert split > 0
+
+
 def test_a_workspace_limit_bounds_the_partials():
     """Whatever the limit, the plan's partials fit it; the limit of the
     allocation-free entry is the library's scratch array."""
@@ -134,3 +187,38 @@ def test_short_chunks_are_as_exact_as_whole_ranges(gpu_device, context, spans, r
             total += float((error ** 2).sum())
         errors.append(total ** 0.5)
     assert errors[0] <= 1.05 * errors[1] and errors[2] == errors[0], errors
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("requests,context,spans,rows,heads", NEWLY_SPLIT)
+def test_newly_split_ranges_are_as_exact_as_whole_ones(gpu_device, requests, context, spans, rows, heads, dtype):
+    """Against fp64, as test_short_chunks_are_as_exact_as_whole_ranges: the chosen
+    plan's error is that of every range whole."""
+
+    dim, (hq, hkv) = 256, heads
+    generator = torch.Generator(device=gpu_device).manual_seed(context)
+    pool = requests * context + 100
+    key, value = (torch.randn(pool, hkv, dim, device=gpu_device, generator=generator).to(dtype) for _ in range(2))
+    perm = torch.randperm(pool, device=gpu_device, generator=generator)
+    table = _rows(context, spans, rows).tolist()
+    lists = [perm[r * context:(r + 1) * context].contiguous() for r in range(requests)]
+    plan_spans = [(slots, int(s), int(s + n)) for slots in lists for _, s, n, _ in table]
+    common = dict(num_q_heads=hq, num_kv_heads=hkv, head_dim=dim)
+    chosen = RepairAttentionPlan(plan_spans, **common)
+    whole = RepairAttentionPlan(plan_spans, split_tokens=8192, **common)
+    query = (1.5 * torch.randn(chosen.num_queries, hq, dim, device=gpu_device, generator=generator)).to(dtype)
+    positions = torch.cat([torch.arange(s, s + n, device=gpu_device) for _, s, n, _ in table])
+    hidden = torch.arange(context, device=gpu_device)[None] > positions[:, None]
+    errors = []
+    for plan in (chosen, whole):
+        got = plan.run(query, key, value).double().view(requests, -1, hq, dim)
+        total = 0.0
+        for request, slots in enumerate(lists):
+            for head in range(hq):
+                k, v = key[slots, head // (hq // hkv)].double(), value[slots, head // (hq // hkv)].double()
+                q = query.view(requests, -1, hq, dim)[request, :, head].double()
+                weights = torch.softmax((q @ k.t() / dim ** 0.5).masked_fill(hidden, float("-inf")), dim=-1)
+                total += float(((got[request, :, head] - weights @ v) ** 2).sum())
+        errors.append(total ** 0.5)
+    assert errors[0] <= 1.05 * errors[1], errors

@@ -1039,6 +1039,14 @@ constexpr double kWidePartialBytesPerTile = 4.5e6;
 // in five chunks.
 constexpr double kSmallCombineTiles = 1.5;
 constexpr double kWideTiles = 1.0;  // five 16-row spans over 3k keys (64/8 heads): 22.1 us at 320 keys, 21.3 at 512
+// The combine's time does not depend on the head dim, the key tile's does: 1.1,
+// 1.4 and 2.15 us at head dims 64, 128 and 256 with a quarter of the compute
+// units busy, where the choice between few and many chunks lies (1.3-1.6, 2.3
+// and 2.9 us with all of them).  With 2.0 and 0.5 for the outer two, as if the
+// tile's time were the head dim's, 300 drawn shapes took the same on average
+// (within 1 %), but single ones up to 31 % more (5 spans over 16k keys, 14/2
+// heads x 256: 51.2 us in 73 items, 39.1 in 37).
+constexpr double combine_scale(int64_t head_dim) { return head_dim == 64 ? 1.3 : head_dim == 256 ? 0.66 : 1.0; }
 constexpr int64_t kRefillTiles = 2;  // an item's slot-list refill (every kDmaMaxRange keys): drain and restart
 // A plan whose cost provably exceeds `beat` returns early with a lower bound
 // of its cost (still above `beat`).
@@ -1047,9 +1055,8 @@ constexpr int64_t kRefillTiles = 2;  // an item's slot-list refill (every kDmaMa
 // 16-bit partial result (all query heads), `wide` says that they are wide,
 // `small` that 512-key chunks leave compute units idle, `chunk_tiles` is the
 // combine's cost per chunk of the most split tile, `combine_scale` the
-// combine's time in key tiles against head dim 128 (a key tile takes 1.3 us
-// there, 2.4 us at head dim 256 and 0.7 us at 64; the combine's time does not
-// depend on it).  A plan whose partials need more than `workspace_limit` bytes (0: no limit)
+// combine's time in key tiles against head dim 128 (combine_scale() below).  A
+// plan whose partials need more than `workspace_limit` bytes (0: no limit)
 // costs HUGE_VAL.
 template <typename Groups>
 double plan_cost_estimate(int64_t split, int64_t num_kv_heads, int64_t partial_bytes, bool wide, bool small,
@@ -1468,7 +1475,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
         const bool wide = dim_known && (candidate < 512 || candidate < whole_keys);
         return plan_cost_estimate(candidate, num_kv_heads, dim_known ? partial_bytes : blind_partial_bytes, wide, small,
                                   dim_known ? kCombineChunkTiles : 0.0,
-                                  dim_known ? 128.0 / static_cast<double>(dim) : 1.0,
+                                  dim_known ? combine_scale(dim) : 1.0,
                                   dim_known ? workspace_limit : 0, beat, [&](auto &&visit) {
           int64_t next_tile = 0;  // a tile's partials count with the first window that holds it
           for (size_t k = 0; k < windows.size(); ++k) {

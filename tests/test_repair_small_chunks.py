@@ -54,6 +54,16 @@ def test_chunks_stay_at_512_where_they_fill_the_device():
     assert _native.repair_attention_plan(table, 28, 4, 0, head_dim=128)[3].split_tokens >= 512
 
 
+def test_the_combine_is_priced_in_the_head_dims_own_tiles():
+    """A key tile of head dim 64 takes 0.8 times that of 128, one of 256 1.5 times
+    (not half and twice): shapes where the difference decides."""
+
+    plan = _native.repair_attention_plan(_rows(15838, 5, 8), 14, 2, 0, head_dim=256)[3]
+    assert plan.split_tokens >= 512 and plan.num_items <= 40  # 39 us; in 73 items of 256 keys 51 us
+    plan = _native.repair_attention_plan(_batch(8, 850, 9, 1), 16, 2, 0, head_dim=64)[3]
+    assert plan.num_items > 16  # 12.3 us in 48 items; in 8 whole ranges 19.3 us
+
+
 @pytest.mark.parametrize("context,spans,rows", [(16384, 15, 16), (8192, 7, 16)])
 def test_head_dim_256_plans_one_round_of_its_two_workgroups_per_window(context, spans, rows):
     items, _, _, info = _native.repair_attention_plan(_rows(context, spans, rows), 8, 4, 0, head_dim=256)

@@ -888,16 +888,16 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
 // together; the running maximum rescales what is summed when a batch raises
 // it.  A partial's weight is its sum l times 2^(m - max): its normalised
 // output O / l then contributes exactly O.
-// Batches `group`, `group` + `groups`, ... only.
-template <int D, typename E, bool kWidePartials>
+// Batches `group`, `group` + kGroups, ... only.
+template <int D, typename E, int kGroups, bool kWidePartials>
 __device__ inline float merge_partials(const AttnParams &p, int first, int count, int h, int c, int part, int group,
-                                       int groups, float &run_max, f32x4 *acc) {
+                                       float &run_max, f32x4 *acc) {
   constexpr int kPer = D / 16;
   constexpr int kBatch = kWidePartials ? 4 : 8;  // (the same registers)
   typedef std::conditional_t<kWidePartials, f32x4, u32x2> Quad;  // four values of a partial's row
   run_max = -INFINITY;
   float total = 0.f;
-  for (int s0 = group * kBatch; s0 < count; s0 += groups * kBatch) {
+  for (int s0 = group * kBatch; s0 < count; s0 += kGroups * kBatch) {
     float ms[kBatch], ls[kBatch];
     Quad rows[kBatch][kPer / 4];
 #pragma unroll
@@ -944,23 +944,13 @@ __device__ inline float merge_partials(const AttnParams &p, int first, int count
 }
 
 // Merges the split partial results of one 16-query tile: workgroup (combine
-// item, query head); thread = (query, 1/16 of the dims), in 1, 2 or 4 groups of
+// item, query head); thread = (query, 1/16 of the dims), in one or two groups of
 // 256 threads that take alternate batches of partials and meet in LDS: a tile's
 // batches otherwise wait for memory one after another, a launch of few
-// workgroups being bound by that latency alone.  One query over 32k keys in 64
-// chunks 23.9 -> 21.3 us, attention included; three spans over 2k keys in 16
-// chunks 16.9 -> 16.2 us.
-template <int D>
-__host__ __device__ constexpr int combine_groups() { return D == 256 ? 2 : 4; }  // most, by registers
-
-template <int D, typename E>
-__global__ void __launch_bounds__(256 * combine_groups<D>()) repair_combine_kernel(const AttnParams p) {
+// workgroups being bound by that latency alone.
+template <int D, typename E, int kGroups>
+__global__ void __launch_bounds__(256 * kGroups) repair_combine_kernel(const AttnParams p) {
   constexpr int kPer = D / 16;
-  // What the other groups merged, given by the launch (none for one group):
-  // per group its sums [kPer / 4][256], then 256 maxima and 256 totals.
-  extern __shared__ __attribute__((aligned(16))) f32x4 other_sums[];
-  auto group_acc = [&](int g) { return other_sums + static_cast<long long>(g) * 256 * (kPer / 4) + g * 128; };
-  auto group_max = [&](int g) { return reinterpret_cast<float *>(group_acc(g) + 256 * (kPer / 4)); };
   const int *ci = p.combine + static_cast<long long>(blockIdx.x) * kCombineInts;
   const int q_index = ci[0], q_count = ci[1] & (kWide - 1), first = ci[2], count = ci[3];
   const bool wide = (ci[1] & kWide) != 0;
@@ -969,39 +959,42 @@ __global__ void __launch_bounds__(256 * combine_groups<D>()) repair_combine_kern
       static_cast<long long>(first) + (wide ? 2ll : 1ll) * count > p.ws_items)
     return;
   const int h = blockIdx.y;
-  const int groups = blockDim.x / 256;
-  const int group = threadIdx.x / 256, thread = threadIdx.x % 256;
+  const int group = kGroups > 1 ? threadIdx.x / 256 : 0, thread = threadIdx.x % 256;
   const int c = thread / 16;
   const int part = thread % 16;
+  if (kGroups == 1 && c >= q_count) return;
   f32x4 acc[kPer / 4];
 #pragma unroll
   for (int d = 0; d < kPer / 4; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   float run_max = -INFINITY, total = 0.f;
   if (c < q_count)
-    total = wide ? merge_partials<D, E, true>(p, first, count, h, c, part, group, groups, run_max, acc)
-                 : merge_partials<D, E, false>(p, first, count, h, c, part, group, groups, run_max, acc);
-  if (groups > 1) {  // uniform
+    total = wide ? merge_partials<D, E, kGroups, true>(p, first, count, h, c, part, group, run_max, acc)
+                 : merge_partials<D, E, kGroups, false>(p, first, count, h, c, part, group, run_max, acc);
+  if constexpr (kGroups > 1) {
+    // What the other groups merged.
+    __shared__ __attribute__((aligned(16))) f32x4 other_acc[kGroups - 1][kPer / 4][256];
+    __shared__ float other_max[kGroups - 1][256], other_total[kGroups - 1][256];
     if (group > 0) {
-      group_max(group - 1)[thread] = run_max;
-      group_max(group - 1)[256 + thread] = total;
+      other_max[group - 1][thread] = run_max;
+      other_total[group - 1][thread] = total;
 #pragma unroll
-      for (int d = 0; d < kPer / 4; ++d) group_acc(group - 1)[256 * d + thread] = acc[d];
+      for (int d = 0; d < kPer / 4; ++d) other_acc[group - 1][d][thread] = acc[d];
     }
     __syncthreads();
     if (group > 0) return;
     float all_max = run_max;
-    for (int g = 0; g + 1 < groups; ++g) all_max = fmaxf(all_max, group_max(g)[thread]);
+    for (int g = 0; g + 1 < kGroups; ++g) all_max = fmaxf(all_max, other_max[g][thread]);
     // A group without partials (or only empty ones) has maximum -inf and sums 0.
     const float scale = run_max == -INFINITY ? 0.f : exp2f(run_max - all_max);
     total *= scale;
 #pragma unroll
     for (int d = 0; d < kPer / 4; ++d) acc[d] *= scale;
-    for (int g = 0; g + 1 < groups; ++g) {
-      const float m = group_max(g)[thread];
+    for (int g = 0; g + 1 < kGroups; ++g) {
+      const float m = other_max[g][thread];
       const float w = m == -INFINITY ? 0.f : exp2f(m - all_max);
-      total += w * group_max(g)[256 + thread];
+      total += w * other_total[g][thread];
 #pragma unroll
-      for (int d = 0; d < kPer / 4; ++d) acc[d] += w * group_acc(g)[256 * d + thread];
+      for (int d = 0; d < kPer / 4; ++d) acc[d] += w * other_acc[g][d][thread];
     }
   }
   if (c >= q_count) return;
@@ -1236,6 +1229,25 @@ void launch_m32(bool f16, dim3 grid, hipStream_t s, const AttnParams &p) {
   else repair_attention_m32_kernel<D, Bf16, kOffsets><<<grid, dim3(m32_threads<D>()), 0, s>>>(p);
 }
 
+// Two groups of threads per workgroup up to one workgroup per compute unit:
+// one query over 32k keys (28 workgroups) 8.6 us with one group, 6.2 with two,
+// 6.0 with four; three 8-row spans over 2k keys (56) 4.6, 4.0, 4.0; 15 spans
+// over 16k keys at head dim 256 (120) 8.2, 6.8.  Beyond that the workgroups
+// themselves hide the latency: 15 spans over 32k keys (392) 6.3, 6.2, 7.5; four
+// 32-row spans over 16k keys (512) 6.8, 6.8, 8.6; 168 spans of 24 requests
+// (2,016) 10.8, 14.7, 22.0.  The rule takes what the plan alone decides, so a
+// plan's results do not depend on the workspace given.
+template <int D>
+void launch_combine(bool f16, dim3 grid, hipStream_t s, const AttnParams &p) {
+  if (static_cast<long long>(grid.x) * grid.y <= kComputeUnits) {
+    if (f16) repair_combine_kernel<D, F16, 2><<<grid, dim3(512), 0, s>>>(p);
+    else repair_combine_kernel<D, Bf16, 2><<<grid, dim3(512), 0, s>>>(p);
+  } else {
+    if (f16) repair_combine_kernel<D, F16, 1><<<grid, dim3(256), 0, s>>>(p);
+    else repair_combine_kernel<D, Bf16, 1><<<grid, dim3(256), 0, s>>>(p);
+  }
+}
+
 // Launches the attention (and the combine of split items) with the partial
 // results in `ws` (ws_items partial slots); the arguments are checked.
 int launch_attention(const ll_repair_attention_args *a, float *ws, long long ws_items, hipStream_t s) {
@@ -1284,25 +1296,9 @@ int launch_attention(const ll_repair_attention_args *a, float *ws, long long ws_
   if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
   if (a->num_combine > 0) {
     const dim3 cgrid(static_cast<unsigned>(a->num_combine), static_cast<unsigned>(a->num_q_heads));
-    // Groups of threads by the average tile's partial slots (a batch takes 8):
-    // one query over 32k keys, 64 slots, 23.9 us with one group and 21.3 with
-    // four; three spans over 2k keys, 32 slots (16 wide partials), 16.9 us with
-    // one, 16.2 with two, 17.4 with four.
-    const long long slots = a->workspace_items / a->num_combine;
-    const int wanted = slots > 32 ? 4 : slots > 8 ? 2 : 1;
-    const auto launch = [&](auto dim, auto f16_kernel, auto bf16_kernel) {
-      constexpr int D = decltype(dim)::value;
-      const int groups = wanted < combine_groups<D>() ? wanted : combine_groups<D>();
-      const size_t lds = static_cast<size_t>(groups - 1) * 256 * (D / 16 + 2) * sizeof(float);
-      if (f16) f16_kernel<<<cgrid, dim3(256 * groups), lds, s>>>(p);
-      else bf16_kernel<<<cgrid, dim3(256 * groups), lds, s>>>(p);
-    };
-    if (a->head_dim == 128)
-      launch(std::integral_constant<int, 128>{}, repair_combine_kernel<128, F16>, repair_combine_kernel<128, Bf16>);
-    else if (a->head_dim == 64)
-      launch(std::integral_constant<int, 64>{}, repair_combine_kernel<64, F16>, repair_combine_kernel<64, Bf16>);
-    else
-      launch(std::integral_constant<int, 256>{}, repair_combine_kernel<256, F16>, repair_combine_kernel<256, Bf16>);
+    if (a->head_dim == 128) launch_combine<128>(f16, cgrid, s, p);
+    else if (a->head_dim == 64) launch_combine<64>(f16, cgrid, s, p);
+    else launch_combine<256>(f16, cgrid, s, p);
     err = hipGetLastError();
     if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
   }

@@ -232,3 +232,33 @@ def test_newly_split_ranges_are_as_exact_as_whole_ones(gpu_device, requests, con
                 total += float(((got[request, :, head] - weights @ v) ** 2).sum())
         errors.append(total ** 0.5)
     assert errors[0] <= 1.05 * errors[1], errors
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("requests,context,spans,rows,heads,dim", [
+    (1, 32768, 1, 1, (28, 4), 128), (1, 8192, 2, 16, (28, 4), 256), (1, 8192, 2, 3, (64, 8), 64),
+    (2, 32768, 5, 32, (28, 4), 128), (12, 12000, 3, 32, (28, 4), 256), (14, 12000, 3, 16, (64, 8), 64),
+])
+def test_the_combine_depends_on_the_plan_alone(gpu_device, requests, context, spans, rows, heads, dim):
+    """Launches of few and of many workgroups (one and two groups of threads
+    each): the same bits with a larger workspace than the plan's, and the whole
+    ranges' result.  Probabilities, partials and outputs are each rounded to
+    2^-9 of themselves, independently per key as the output's own terms are, in
+    either run: 2^-7 of the output's norm for all four."""
+
+    generator = torch.Generator(device=gpu_device).manual_seed(context + dim)
+    pool, (hq, hkv) = requests * context + 64, heads
+    key, value = (torch.randn(pool, hkv, dim, device=gpu_device, generator=generator).bfloat16() for _ in range(2))
+    perm = torch.randperm(pool, device=gpu_device, generator=generator)
+    plan_spans = [(perm[r * context:(r + 1) * context].contiguous(), int(s), int(s + n))
+                  for r in range(requests) for _, s, n, _ in _rows(context, spans, rows).tolist()]
+    common = dict(num_q_heads=hq, num_kv_heads=hkv, head_dim=dim)
+    plan = RepairAttentionPlan(plan_spans, split_tokens=640, **common)
+    query = torch.randn(plan.num_queries, hq, dim, device=gpu_device, generator=generator).bfloat16()
+    assert plan.info["num_combine"] > 0 and int(plan.combine[3::4].max()) > 8
+    got = plan.run(query, key, value)
+    plan.info["workspace_items"] *= 9
+    plan.workspace = torch.empty(9 * plan.workspace.numel(), device=gpu_device)
+    assert torch.equal(plan.run(query, key, value), got)
+    whole = RepairAttentionPlan(plan_spans, split_tokens=32768, **common).run(query, key, value)
+    assert float((got.double() - whole.double()).norm()) <= 2.0 ** -7 * float(whole.double().norm())

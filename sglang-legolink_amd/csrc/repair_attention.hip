@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
     return field < kWave ? lo : hi;
   };
   const int kv_off = it(0), kv_begin = it(1), kv_end = it(2), n_tiles = it(3);
-  const int pair_first = it(4), pair_count = it(5) & (kWide - 1);
+  const int pair_first = it(4), pair_count = it(5) & ~kWide;
   const bool wide = (it(5) & kWide) != 0;
   // blockIdx.y = (KV head, pair chunk): this workgroup's pairs of the window
   // are [wg_first, wg_end), counted from the item's first tile.
@@ -478,9 +478,8 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   auto load_first_slots = [&](int chunk_begin) __attribute__((always_inline)) {
     load_slots(chunk_begin, tid, !kLeadFromList);
   };
-  if (load_stop <= kv_begin) load_stop = kv_begin;  // no keys: no slots, no tiles
-  else
-  load_first_slots(kv_begin);
+  if (load_stop > kv_begin) load_first_slots(kv_begin);
+  else load_stop = kv_begin;  // no keys: no slots, no tiles
 
   // The wave's two pairs; a pair computes when its tile and head exist and its
   // table entry is sane.
@@ -952,7 +951,7 @@ template <int D, typename E, int kGroups>
 __global__ void __launch_bounds__(256 * kGroups) repair_combine_kernel(const AttnParams p) {
   constexpr int kPer = D / 16;
   const int *ci = p.combine + static_cast<long long>(blockIdx.x) * kCombineInts;
-  const int q_index = ci[0], q_count = ci[1] & (kWide - 1), first = ci[2], count = ci[3];
+  const int q_index = ci[0], q_count = ci[1] & ~kWide, first = ci[2], count = ci[3];
   const bool wide = (ci[1] & kWide) != 0;
   if (q_count < 1 || q_count > kQueries || q_index < 0 ||
       static_cast<long long>(q_index) + q_count > p.num_queries || first < 0 || count < 1 ||

@@ -262,3 +262,32 @@ def test_the_combine_depends_on_the_plan_alone(gpu_device, requests, context, sp
     assert torch.equal(plan.run(query, key, value), got)
     whole = RepairAttentionPlan(plan_spans, split_tokens=32768, **common).run(query, key, value)
     assert float((got.double() - whole.double()).norm()) <= 2.0 ** -7 * float(whole.double().norm())
+
+
+@pytest.mark.gpu
+def test_counts_with_other_bits_than_the_wide_flag_are_refused(gpu_device):
+    """An item or combine item whose count is none (negative, or with bits above
+    the flag) is skipped, as without the flag: its output stays as it was."""
+
+    slots = torch.randperm(2000, device=gpu_device)
+    key, value = (torch.randn(2000, 4, 128, device=gpu_device).bfloat16() for _ in range(2))
+    plan = RepairAttentionPlan([(slots, 1900, 1916)], num_q_heads=28, num_kv_heads=4, head_dim=128)
+    query = torch.randn(16, 28, 128, device=gpu_device).bfloat16()
+    good = plan.run(query, key, value)
+    assert plan.info["num_combine"] == 1 and int(plan.combine[1]) == 16 | WIDE
+    for change in (1 << 9, 1 << 20, -1 << 31):
+        plan.combine[1] ^= change
+        untouched = torch.full_like(good, 7.0)
+        plan.run(query, key, value, output=untouched)
+        assert bool((untouched == 7.0).all())
+        plan.combine[1] ^= change
+    whole = RepairAttentionPlan([(slots, 100, 116)], num_q_heads=28, num_kv_heads=4, head_dim=128, split_tokens=512)
+    assert whole.info["num_combine"] == 0
+    counts = whole.items.view(-1, _native.REPAIR_ITEM_INTS)[:, 5]
+    for change in (1 << 9, 1 << 20, -1 << 31):
+        counts ^= change
+        untouched = torch.full_like(good, 7.0)
+        whole.run(query, key, value, output=untouched)
+        assert bool((untouched == 7.0).all())
+        counts ^= change
+    assert torch.equal(plan.run(query, key, value), good)

@@ -10,7 +10,11 @@
 // (kv_link._eligibility, PreparedKVScatter) and the block is filled, and False
 // otherwise, with nothing to rely on in it: the caller then runs the Python
 // checks, which name the reason.  Only plain tensors are taken here.
+//
+// The module names the torch version and the block sizes that it was built
+// for: the caller uses it only where they are its own.
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cstdint>
 #include <cstring>
@@ -224,4 +228,14 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_link_arguments", "Link argument b
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__link_arguments(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__link_arguments(void) {
+  PyObject *created = PyModule_Create(&module);
+  if (created == nullptr) return nullptr;
+  if (PyModule_AddStringConstant(created, "TORCH_VERSION", TORCH_VERSION) != 0 ||
+      PyModule_AddIntConstant(created, "LINK_ARGS_SIZE", sizeof(ll_kv_link_args)) != 0 ||
+      PyModule_AddIntConstant(created, "SCATTER_ARGS_SIZE", sizeof(ll_kv_scatter_args)) != 0) {
+    Py_DECREF(created);
+    return nullptr;
+  }
+  return created;
+}

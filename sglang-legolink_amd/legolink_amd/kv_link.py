@@ -26,11 +26,24 @@ import torch
 
 from . import _native
 
-try:
-    from . import _link_arguments
-except ImportError as error:
-    raise ImportError("legolink_amd._link_arguments is not built: run `python -m legolink_amd.build` "
-                      "(or __graft_entry__.build())") from error
+
+
+def _load_link_arguments() -> Any:
+    """The native check-and-fill of argument blocks, or None where it is not
+    built or was built for another torch or other argument blocks: it reads
+    tensors through torch's C++ classes and writes the blocks by offset.  The
+    Python checks then take every call, with the same result."""
+
+    try:
+        from . import _link_arguments as module
+    except ImportError:
+        return None
+    built_for = tuple(getattr(module, name, None) for name in ("TORCH_VERSION", "LINK_ARGS_SIZE", "SCATTER_ARGS_SIZE"))
+    here = (torch.__version__.split("+")[0], ctypes.sizeof(_native.LinkArgs), ctypes.sizeof(_native.ScatterArgs))
+    return module if built_for == here else None
+
+
+_link_arguments = _load_link_arguments()
 
 # Reason reported when the HIP library cannot be loaded; the reference reports
 # "triton_not_installed" in the same position (legolink_triton.py:174-175).
@@ -538,7 +551,7 @@ class PreparedKVLink:
         # checks run where it declines, and name the reason.
         args = _native.LinkArgs()
         tables = (ctypes.c_void_p * ((4 if source_key_buffers else 2) * len(key_buffers)))()
-        filled = _native.library_available() and _link_arguments.fill_link(
+        filled = _link_arguments is not None and _native.library_available() and _link_arguments.fill_link(
             ctypes.addressof(args), ctypes.addressof(tables), key_buffers, value_buffers, source_key_buffers,
             source_value_buffers, source_slots, destination_slots, local_positions, global_positions,
             cos_sin_cache, repair_mask, int(rotary_dim))
@@ -875,8 +888,10 @@ class PreparedKVScatter:
         args.struct_size = ctypes.sizeof(_native.ScatterArgs)
         tables = (ctypes.c_void_p * (2 * layers))()
         self._tables = (tables,)
-        if not _link_arguments.fill_scatter(ctypes.addressof(args), ctypes.addressof(tables), key_buffers,
-                                            value_buffers, destination_slots, repaired_keys, repaired_values):
+        filled = _link_arguments is not None and _link_arguments.fill_scatter(
+            ctypes.addressof(args), ctypes.addressof(tables), key_buffers, value_buffers, destination_slots,
+            repaired_keys, repaired_values)
+        if not filled:
             if not all(tensor.is_cuda and tensor.device == key_buffer.device for tensor in tensors):
                 _raise_unavailable("cuda_tensors_required")
             for key, value in zip(key_buffers, value_buffers, strict=True):

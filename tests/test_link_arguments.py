@@ -5,6 +5,10 @@ fills what they fill."""
 from __future__ import annotations
 
 import ctypes
+import os
+import subprocess
+import sys
+from pathlib import Path
 
 import pytest
 import torch
@@ -141,6 +145,73 @@ def test_native_fill_declines_what_is_no_tensor_list():
         assert not _fill(broken)[0], name
     assert not _link_arguments.fill_link()
     assert not _link_arguments.fill_scatter(0, 0, [], [], None, None, None)
+
+
+_IMPORT_WITHOUT = """
+import sys, types
+import torch
+name = "legolink_amd._link_arguments"
+if {sizes!r} is None:
+    sys.modules[name] = None  # as if it were not built
+else:
+    sys.modules[name] = module = types.ModuleType(name)
+    if {sizes!r}:
+        module.TORCH_VERSION, module.LINK_ARGS_SIZE, module.SCATTER_ARGS_SIZE = {sizes!r}
+    module.fill_link = module.fill_scatter = None  # never called
+from legolink_amd import kv_link
+assert kv_link._link_arguments is None
+buffer, index = torch.zeros(8, 2, 64, dtype=torch.bfloat16), torch.arange(4)
+print(kv_link.check_fused_kv_link_eligibility(
+    key_buffer=buffer, value_buffer=buffer, source_slots=index, destination_slots=index, local_positions=index,
+    global_positions=index, cos_sin_cache=torch.zeros(8, 64), rotary_dim=64).reason)
+"""
+
+
+@pytest.mark.parametrize("sizes", [None, (), ("1.0.0", None, None), (None, 8, None), (None, None, 1 << 20)])
+@pytest.mark.parametrize("library,reason", [(None, "cuda_tensors_required"), ("/nowhere/lib.so", "hip_kv_link_not_built")])
+def test_operator_imports_without_a_matching_module(sizes, library, reason):
+    """An unbuilt tree, another torch or other argument blocks: the operator
+    imports, keeps its reasons and takes the Python checks."""
+
+    if sizes:
+        own = (_link_arguments.TORCH_VERSION, ctypes.sizeof(_native.LinkArgs), ctypes.sizeof(_native.ScatterArgs))
+        sizes = tuple(value if other is None else other for value, other in zip(own, sizes))
+    package = Path(kv_link.__file__).resolve().parents[1]
+    environment = {**os.environ, "PYTHONPATH": str(package)}
+    if library is not None:
+        environment["LEGOLINK_KV_LIBRARY"] = library
+    done = subprocess.run([sys.executable, "-c", _IMPORT_WITHOUT.format(sizes=sizes)], env=environment,
+                          capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr
+    assert done.stdout.strip() == reason
+
+
+def test_the_built_module_is_the_one_in_use():
+    assert kv_link._link_arguments is _link_arguments
+    assert _link_arguments.LINK_ARGS_SIZE == ctypes.sizeof(_native.LinkArgs)
+    assert _link_arguments.SCATTER_ARGS_SIZE == ctypes.sizeof(_native.ScatterArgs)
+    assert torch.__version__.split("+")[0] == _link_arguments.TORCH_VERSION
+
+
+@pytest.mark.gpu
+def test_python_checks_alone_link_and_write_back_the_same(gpu_device, monkeypatch):
+    results = []
+    for module in (_link_arguments, None):
+        monkeypatch.setattr(kv_link, "_link_arguments", module)
+        torch.manual_seed(3)
+        inputs = _inputs(gpu_device, vdim=32)
+        for buffer in (*inputs["keys"], *inputs["values"]):
+            buffer.normal_()
+        kv_link.fused_kv_link_layers_inplace(
+            key_buffers=inputs["keys"], value_buffers=inputs["values"], source_slots=inputs["src"],
+            destination_slots=inputs["dst"], local_positions=inputs["local"], global_positions=inputs["global"],
+            cos_sin_cache=inputs["table"], prefix_token_count=2, rotary_dim=64, is_neox_style=True)
+        rows = torch.ones(3, 5, 2, 64, dtype=torch.bfloat16, device=gpu_device)
+        kv_link.scatter_kv_rows_inplace(
+            key_buffers=inputs["keys"], value_buffers=inputs["values"], destination_slots=inputs["src"][:5],
+            repaired_keys=rows, repaired_values=rows[..., :32].contiguous())
+        results.append(torch.cat([buffer.flatten() for buffer in (*inputs["keys"], *inputs["values"])]))
+    assert torch.equal(*results)
 
 
 class _Subclass(torch.Tensor):

@@ -18,6 +18,7 @@ reference's concatenation restricted to each set, in the same order.
 
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -260,6 +261,15 @@ def order_link_maps(maps: torch.Tensor, mask: Optional[torch.Tensor], *, key_row
     entries within the buckets too (``ll_order_link_maps_exact``; at most
     ``_native.ORDER_EXACT_SLOTS`` slots)."""
 
+    return _order(maps, mask, key_row, prefix, num_slots, workspace, _native.stream_handle(stream, maps.device),
+                  stream, exact)
+
+
+def _order(maps: torch.Tensor, mask: Optional[torch.Tensor], key_row: int, prefix: int, num_slots: int,
+           workspace: torch.Tensor, handle: int, stream: torch.cuda.Stream | None,
+           exact: bool) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """``order_link_maps`` on the stream of ``handle`` (``stream``, or with None the current one)."""
+
     if key_row not in (0, 1):
         raise ValueError("key_row must be 0 (source slots) or 1 (destination slots)")
     n = int(maps.shape[1])
@@ -287,11 +297,48 @@ def order_link_maps(maps: torch.Tensor, mask: Optional[torch.Tensor], *, key_row
             if scratch_mask is not None:
                 scratch_mask.record_stream(stream)
         _native.order_link_maps_exact(args, scratch.data_ptr(),
-                                      None if scratch_mask is None else scratch_mask.data_ptr(),
-                                      _native.stream_handle(stream, maps.device))
+                                      None if scratch_mask is None else scratch_mask.data_ptr(), handle)
     else:
-        _native.order_link_maps(args, _native.stream_handle(stream, maps.device))
+        _native.order_link_maps(args, handle)
     return out, out_mask
+
+
+class OrderWorkspaces:
+    """The workspaces of ``order_link_maps`` on the current streams: one per
+    stream, made when first needed and zero between calls.  A call's launches
+    are enqueued under a lock, so that threads that share a stream do not mix
+    theirs; under stream capture a call takes a workspace of its own, since the
+    graph's replays may overlap later calls."""
+
+    LIMIT = 64  # streams whose workspace (128 KB each) is kept
+
+    def __init__(self) -> None:
+        self._lock = threading.Lock()
+        self._kept: dict[tuple[Optional[int], int], torch.Tensor] = {}
+
+    def order(self, maps: torch.Tensor, mask: Optional[torch.Tensor], *, key_row: int, prefix: int, num_slots: int,
+              exact: bool = False) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
+        """``order_link_maps`` on the current stream of the maps' device."""
+
+        device = maps.device
+        handle = _native.stream_handle(None, device)
+        if torch.cuda.is_current_stream_capturing():
+            return _order(maps, mask, key_row, prefix, num_slots, self._zeros(device), handle, None, exact)
+        key = (device.index, handle)
+        with self._lock:
+            # Out of the table during the call: one that fails half-way leaves
+            # counters behind and is not used again.
+            workspace = self._kept.pop(key, None)
+            if workspace is None:
+                workspace = self._zeros(device)
+            ordered = _order(maps, mask, key_row, prefix, num_slots, workspace, handle, None, exact)
+            if len(self._kept) < self.LIMIT:
+                self._kept[key] = workspace
+        return ordered
+
+    @staticmethod
+    def _zeros(device: torch.device) -> torch.Tensor:
+        return torch.zeros(_native.ORDER_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
 
 
 def order_by_destination(maps: torch.Tensor, mask: Optional[torch.Tensor], *, prefix: int, num_slots: int,

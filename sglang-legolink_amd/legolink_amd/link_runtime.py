@@ -39,6 +39,7 @@ Differences from the reference that keep the result identical:
 
 from __future__ import annotations
 
+import functools
 import itertools
 import operator
 import os
@@ -423,7 +424,8 @@ class PreparedLink:
                  layer_groups_per_block: int = 0, order_by_source: Optional[bool] = None,
                  fused_mode: str = "required", delta_staging: str = "auto",
                  skipped_rows: Optional[torch.Tensor] = None, visit_order: Optional[str] = None,
-                 order_workspace: Optional[torch.Tensor] = None) -> None:
+                 order_workspace: Optional[torch.Tensor] = None,
+                 order_workspaces: Optional[link_maps.OrderWorkspaces] = None) -> None:
         self.pool = pool
         self.layers = layers
         self.maps = maps
@@ -480,10 +482,11 @@ class PreparedLink:
         self.stream_source_rows = (maps.request_count == 1 and not self.order_by_source
                                    and token_count * len(layers) * row_bytes > MEMORY_SIDE_CACHE_BYTES)
         sort_row = {"source": 0, "destination": 1}.get(self.visit_order)
-        # Batches keep their own: they may be prepared on several streams at once.
-        if sort_row == 0 or (sort_row == 1 and order_workspace is None):
-            order_workspace = torch.zeros(_native.ORDER_WORKSPACE_BYTES, dtype=torch.uint8,
-                                          device=key_buffers[0].device)
+        # A workspace given is the caller's to keep to one stream.
+        if order_workspace is not None:
+            order_maps = functools.partial(link_maps.order_link_maps, workspace=order_workspace)
+        else:
+            order_maps = (order_workspaces or link_maps.OrderWorkspaces()).order
         # delta_staging "table": a layer-major value pass writes every token's
         # RoPE delta to a table and a layer-major key pass reads it back
         # (measured 1.4-2.0 % slower than the default staged deltas on c2,
@@ -531,9 +534,9 @@ class PreparedLink:
                 # Source order is exact (one launch more): a batch's repeated
                 # source rows must be adjacent to hit in cache (bucketed, c3's
                 # link ran 2.7-3.6 % slower: 8.59-8.65 against 8.35-8.39 ms).
-                device_maps, mask = link_maps.order_link_maps(
+                device_maps, mask = order_maps(
                     device_maps, mask.view(torch.uint8) if mask is not None else None, key_row=sort_row,
-                    prefix=prefix, num_slots=order_slots, workspace=order_workspace, exact=sort_row == 0)
+                    prefix=prefix, num_slots=order_slots, exact=sort_row == 0)
                 self._kernel_maps.append(device_maps)
             elif (sort_row is not None or eager_entries is not None) and count - prefix > 1:
                 tail = device_maps[:, prefix:]
@@ -696,7 +699,7 @@ class KVLinkExecutor:
         self.arena = arena
         self.count_skipped_rows = bool(count_skipped_rows)
         self._skip_counters: dict[torch.device, torch.Tensor] = {}
-        self._order_workspaces: dict[torch.device, torch.Tensor] = {}
+        self._order_workspaces = link_maps.OrderWorkspaces()
 
     @property
     def layers(self) -> list[int]:
@@ -711,17 +714,6 @@ class KVLinkExecutor:
             counter = torch.zeros(1, dtype=torch.int64, device=device)
             self._skip_counters[device] = counter
         return counter
-
-    def _order_workspace(self, device: torch.device) -> torch.Tensor:
-        """The zeroed workspace of the destination ordering on ``device``,
-        shared by this executor's links (prepared on one stream)."""
-
-        device = torch.device(device)
-        workspace = self._order_workspaces.get(device)
-        if workspace is None:
-            workspace = torch.zeros(_native.ORDER_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
-            self._order_workspaces[device] = workspace
-        return workspace
 
     def skipped_rows(self, *, reset: bool = True) -> int:
         """Tokens the links so far skipped because a slot or position was out
@@ -908,7 +900,7 @@ class KVLinkExecutor:
             validate_indices=validate_indices, arena=self.arena,
             layer_groups_per_block=self.layer_groups_per_block, fused_mode=self._fused_mode(),
             delta_staging=self.delta_staging, skipped_rows=self._skip_counter(device),
-            visit_order=self.visit_order, order_workspace=self._order_workspace(device),
+            visit_order=self.visit_order, order_workspaces=self._order_workspaces,
         )
         prepared.host_prepare_s = time.perf_counter() - started
         return prepared
@@ -944,7 +936,7 @@ class KVLinkExecutor:
             fused_mode=self._fused_mode(), delta_staging=self.delta_staging,
             skipped_rows=self._skip_counter(device),
             visit_order=None if order_by_source is not None else self.visit_order,
-            order_workspace=self._order_workspace(device),
+            order_workspaces=self._order_workspaces,
         )
         prepared.host_prepare_s = time.perf_counter() - started
         return prepared

@@ -1235,6 +1235,73 @@ __global__ void __launch_bounds__(kOrderThreads) order_small_kernel(const OrderP
   }
 }
 
+// The count and the scatter of an exact order: a workgroup gathers its own run
+// of entries by bucket in LDS first, so that a bucket's global counter takes one
+// atomic per workgroup instead of one per entry.  A batch's requests read the
+// same catalogue blocks, whose slots often lie side by side: with an atomic per
+// entry they pile up on few counters, which take them one after another (24
+// requests of the same 8 contiguous blocks x 512 in a pool of 1,048,576 rows:
+// 711 us for the whole order -> 41, torch's argsort and gather 77; with slots
+// scattered over the pool 33 -> 36).  No layout measured, 4 to 256 requests in
+// pools of 16,384 to 1,048,576 rows, takes longer than torch's.
+constexpr int kOrderRunBlocks = 512;  // two workgroups per compute unit (64 KB of LDS each)
+
+__device__ __forceinline__ void order_own_run(const OrderParams &p, long long &begin, long long &end) {
+  const long long chunks = (p.count + kOrderThreads - 1) / kOrderThreads;
+  const long long run = (chunks + gridDim.x - 1) / gridDim.x * kOrderThreads;
+  begin = min(blockIdx.x * run, p.count);
+  end = min(begin + run, p.count);
+}
+
+// The run's entries [begin, end) by bucket, in LDS.
+__device__ __forceinline__ void order_count_run(const OrderParams &p, long long begin, long long end, int *places) {
+#pragma unroll
+  for (int k = 0; k < kOrderBuckets / kOrderThreads; ++k) places[k * kOrderThreads + threadIdx.x] = 0;
+  __syncthreads();
+  for (long long i = begin + threadIdx.x; i < end; i += kOrderThreads)
+    if (i >= p.prefix) atomicAdd(&places[order_bucket(p.key[i], p)], 1);
+  __syncthreads();
+}
+
+__global__ void __launch_bounds__(kOrderThreads) order_count_run_kernel(const OrderParams p) {
+  __shared__ int places[kOrderBuckets];
+  long long begin, end;
+  order_own_run(p, begin, end);
+  order_count_run(p, begin, end, places);
+#pragma unroll
+  for (int k = 0; k < kOrderBuckets / kOrderThreads; ++k) {
+    const int b = k * kOrderThreads + threadIdx.x;
+    const int own = places[b];
+    if (own > 0) atomicAdd(&p.counts[b], own);
+  }
+}
+
+__global__ void __launch_bounds__(kOrderThreads) order_scatter_run_kernel(const OrderParams p) {
+  __shared__ int places[kOrderBuckets];  // the run's counts, then its next places
+  const long long n = p.count - p.prefix;
+  long long begin, end;
+  order_own_run(p, begin, end);
+  order_count_run(p, begin, end, places);
+#pragma unroll
+  for (int k = 0; k < kOrderBuckets / kOrderThreads; ++k) {
+    const int b = k * kOrderThreads + threadIdx.x;
+    const int own = places[b];
+    if (own > 0) places[b] = atomicAdd(&p.offsets[b], own);
+  }
+  __syncthreads();
+  for (long long i = begin + threadIdx.x; i < end; i += kOrderThreads) {
+    long long o = i;
+    if (i >= p.prefix) {
+      const long long place = atomicAdd(&places[order_bucket(p.key[i], p)], 1);
+      if (place < 0 || place >= n) continue;  // only if the workspace was shared by overlapping calls
+      o = p.prefix + place;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p.out[r * p.cap + o] = p.maps[r * p.cap + i];
+    if (p.mask != nullptr) p.out_mask[o] = p.mask[i];
+  }
+}
+
 // Exact order within the buckets: one wave per bucket (the entries that the
 // scatter left in [offsets[b - 1], offsets[b]) of the tail of `maps`) counts its
 // entries by slot, scans the counts across its lanes and writes every entry to
@@ -1243,7 +1310,7 @@ __global__ void __launch_bounds__(kOrderThreads) order_small_kernel(const OrderP
 // A batched link wants its repeated source rows next to each other: buckets
 // alone leave them up to 64 slots apart, which costs c3's link 3 %, and
 // torch's argsort and the gather of its result take 12 launches.  24 requests
-// x 4,096 tokens: 72 us (argsort and gather) -> 32 us in all four launches, the
+// x 4,096 tokens: 72 us (argsort and gather) -> 37 us in all four launches, the
 // batch's link as a whole 1,691 -> 1,655 us.  Latency-bound: a few entries per
 // wave, 64 bytes read and written per entry.
 constexpr int kOrderExactSlots = kWave;
@@ -1263,8 +1330,17 @@ __global__ void __launch_bounds__(kOrderExactWaves * kWave) order_within_buckets
   __syncthreads();
   const int slot_mask = (1 << p.shift) - 1;
   const long long *key = p.key + p.prefix;
-  for (long long i = begin + lane; i < end; i += kWave)
-    atomicAdd(&place[static_cast<int>(key[i]) & slot_mask], 1);
+  // Four rounds' keys (and, below, entries) are requested together: a bucket of
+  // a block that hundreds of requests link holds thousands of entries.
+  constexpr int kAhead = 4;
+  for (long long i = begin + lane; i < end; i += kAhead * kWave) {
+    long long slot[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) slot[u] = key[min(i + u * kWave, end - 1)];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (i + u * kWave < end) atomicAdd(&place[static_cast<int>(slot[u]) & slot_mask], 1);
+  }
   __syncthreads();
   const int own = place[lane];
   int inclusive = own;
@@ -1276,11 +1352,26 @@ __global__ void __launch_bounds__(kOrderExactWaves * kWave) order_within_buckets
   __syncthreads();
   place[lane] = inclusive - own;
   __syncthreads();
-  for (long long i = begin + lane; i < end; i += kWave) {
-    const long long o = p.prefix + begin + atomicAdd(&place[static_cast<int>(key[i]) & slot_mask], 1);
+  const long long *maps = p.maps + p.prefix;
+  for (long long i = begin + lane; i < end; i += kAhead * kWave) {
+    long long slot[kAhead], entry[kAhead][4];
+    unsigned char mask_byte[kAhead];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) p.out[r * p.cap + o] = p.maps[r * p.cap + p.prefix + i];
-    if (p.mask != nullptr) p.out_mask[o] = p.mask[p.prefix + i];
+    for (int u = 0; u < kAhead; ++u) {
+      const long long e = min(i + u * kWave, end - 1);
+      slot[u] = key[e];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) entry[u][r] = maps[r * p.cap + e];
+      if (p.mask != nullptr) mask_byte[u] = p.mask[p.prefix + e];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (i + u * kWave >= end) continue;
+      const long long o = p.prefix + begin + atomicAdd(&place[static_cast<int>(slot[u]) & slot_mask], 1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p.out[r * p.cap + o] = entry[u][r];
+      if (p.mask != nullptr) p.out_mask[o] = mask_byte[u];
+    }
   }
   // The identity prefix stays in place.
   for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < p.prefix;
@@ -2388,9 +2479,11 @@ static int order_link_maps(const ll_order_maps_args *a, int64_t *scratch_maps, u
     if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
     return LL_OK;
   }
+  const int64_t runs = std::min<int64_t>((a->count + kOrderThreads - 1) / kOrderThreads, kOrderRunBlocks);
   if (tail > 0) {
     const int64_t blocks = (tail + 255) / 256;
-    order_count_kernel<<<dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s>>>(p);
+    if (exact) order_count_run_kernel<<<dim3(static_cast<unsigned>(runs)), dim3(kOrderThreads), 0, s>>>(p);
+    else order_count_kernel<<<dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
     order_offsets_kernel<<<dim3(1), dim3(kOrderThreads), 0, s>>>(p);
@@ -2398,7 +2491,8 @@ static int order_link_maps(const ll_order_maps_args *a, int64_t *scratch_maps, u
     if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
   }
   const int64_t blocks = (a->count + 255) / 256;
-  order_scatter_kernel<<<dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s>>>(p);
+  if (exact) order_scatter_run_kernel<<<dim3(static_cast<unsigned>(runs)), dim3(kOrderThreads), 0, s>>>(p);
+  else order_scatter_kernel<<<dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s>>>(p);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return fail(LL_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
   if (refine) {

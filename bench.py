@@ -1140,7 +1140,7 @@ def main() -> int:
         "launch": launch,
         "roofline": {
             "bound": "hbm",
-            "kernel": "kv_link_vec_kernel" if launch["kernel"] == "vector" else "kv_link_generic_kernel",
+            "kernel": launch["kernel_name"],
             "achieved": round(achieved, 2),
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",

@@ -62,7 +62,8 @@ enum {
 
 /* Kernel selection (ll_kv_link_args.kernel). */
 enum {
-  LL_KERNEL_AUTO = 0,   /* vectorised kernel when the shape allows, else generic */
+  LL_KERNEL_AUTO = 0,   /* vectorised kernel when the shape allows, else generic: by 16-byte chunks where
+                           head dims and rotary halves are whole chunks, else element-wise */
   LL_KERNEL_VECTOR = 1, /* 16-byte row-chunk kernel; LL_ERR_UNSUPPORTED_KERNEL if the shape does not fit */
   LL_KERNEL_GENERIC = 2 /* element-wise kernel for every eligible shape */
 };
@@ -605,7 +606,8 @@ int64_t ll_repair_scratch_bytes(void);
 
 /* Which kernel and launch shape ll_kv_link would use (no GPU work). */
 typedef struct ll_launch_info {
-  int64_t kernel;                  /* LL_KERNEL_VECTOR or LL_KERNEL_GENERIC */
+  int64_t kernel;                  /* LL_KERNEL_VECTOR or LL_KERNEL_GENERIC (ll_kv_link_kernel_name tells
+                                      the chunk kernel from the element-wise one) */
   int64_t launches;                /* kernel launches (one per group of <= 64 layers) */
   int64_t grid_x;                  /* of the first launch */
   int64_t grid_y;
@@ -617,6 +619,11 @@ typedef struct ll_launch_info {
 
 int ll_kv_link(const ll_kv_link_args *args, ll_stream_t stream);
 int ll_kv_link_describe(const ll_kv_link_args *args, ll_launch_info *info);
+/* Name of the kernel that ll_kv_link would launch: "kv_link_vec_kernel",
+ * "kv_link_layer_kernel" (LL_DELTA_TABLE), "kv_link_chunk_kernel" or
+ * "kv_link_generic_kernel" (both LL_KERNEL_GENERIC in ll_launch_info.kernel);
+ * NULL where ll_kv_link_describe fails. */
+const char *ll_kv_link_kernel_name(const ll_kv_link_args *args);
 int ll_kv_scatter_rows(const ll_kv_scatter_args *args, ll_stream_t stream);
 int ll_kv_build_link_maps(const ll_link_maps_args *args, ll_stream_t stream);
 

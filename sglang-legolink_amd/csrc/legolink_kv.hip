@@ -1521,8 +1521,8 @@ struct LinkPlan {
   bool chunked;  // LL_KERNEL_GENERIC by the chunk kernel
   int block_threads;
   long long grid_x;
-  int layers_per_wave;  // vector kernel
-  int layer_groups_per_block;  // vector kernel
+  int layers_per_wave;  // vector and chunk kernels (else 1)
+  int layer_groups_per_block;  // vector kernel (else 1)
   long long key_waves;  // chunk kernel
   int launches;
   bool staged;  // vector kernel: workgroup-staged deltas
@@ -1899,6 +1899,13 @@ int ll_kv_link_describe(const ll_kv_link_args *args, ll_launch_info *info) {
                             : (plan.layer_major ? LL_DELTA_TABLE : (plan.staged ? LL_DELTA_WORKGROUP : LL_DELTA_PER_WAVE));
   if (plan.layer_major) info->grid_y = 1;
   return LL_OK;
+}
+
+const char *ll_kv_link_kernel_name(const ll_kv_link_args *args) {
+  LinkPlan plan;
+  if (validate_link(args) != LL_OK || plan_link(args, &plan) != LL_OK) return nullptr;
+  if (plan.kernel == LL_KERNEL_VECTOR) return plan.layer_major ? "kv_link_layer_kernel" : "kv_link_vec_kernel";
+  return plan.chunked ? "kv_link_chunk_kernel" : "kv_link_generic_kernel";
 }
 
 int ll_kv_link(const ll_kv_link_args *a, ll_stream_t stream) {

@@ -56,6 +56,7 @@ LL_ERR_HIP = -20
 EXPORTED_SYMBOLS = (
     "ll_kv_link",
     "ll_kv_link_describe",
+    "ll_kv_link_kernel_name",
     "ll_kv_scatter_rows",
     "ll_status_reason",
     "ll_last_error",
@@ -366,6 +367,8 @@ def load_library() -> ctypes.CDLL:
         lib.ll_kv_link.restype = ctypes.c_int
         lib.ll_kv_link_describe.argtypes = [ctypes.POINTER(LinkArgs), ctypes.POINTER(LaunchInfo)]
         lib.ll_kv_link_describe.restype = ctypes.c_int
+        lib.ll_kv_link_kernel_name.argtypes = [ctypes.POINTER(LinkArgs)]
+        lib.ll_kv_link_kernel_name.restype = ctypes.c_char_p
         lib.ll_kv_scatter_rows.argtypes = [ctypes.POINTER(ScatterArgs), _ptr]
         lib.ll_kv_scatter_rows.restype = ctypes.c_int
         lib.ll_status_reason.argtypes = [ctypes.c_int]
@@ -465,6 +468,14 @@ def kv_link_describe(args: LinkArgs) -> LaunchInfo:
     info = LaunchInfo()
     _check(load_library().ll_kv_link_describe(ctypes.byref(args), ctypes.byref(info)))
     return info
+
+
+def kv_link_kernel_name(args: LinkArgs) -> str | None:
+    """The kernel that the link would launch (None for arguments it would refuse)."""
+
+    args.struct_size = ctypes.sizeof(LinkArgs)
+    name = load_library().ll_kv_link_kernel_name(ctypes.byref(args))
+    return None if name is None else name.decode()
 
 
 def kv_build_link_maps(args: LinkMapsArgs, stream: int) -> None:

@@ -95,7 +95,7 @@ def delta_workspace_bytes(token_count: int, rotary_dim: int) -> int:
 _DELTA_NAMES = {code: name for name, code in DELTA_STAGINGS.items()}
 
 
-def _launch_record(info: _native.LaunchInfo) -> dict[str, Any]:
+def _launch_record(args: _native.LinkArgs, info: _native.LaunchInfo) -> dict[str, Any]:
     return {
         "kernel": "vector" if info.kernel == _native.KERNEL_VECTOR else "generic",
         "launches": int(info.launches),
@@ -105,6 +105,7 @@ def _launch_record(info: _native.LaunchInfo) -> dict[str, Any]:
         "layers_per_wave": int(info.layers_per_wave),
         "layer_groups_per_block": int(info.layer_groups_per_block),
         "delta_staging": _DELTA_NAMES.get(int(info.delta_staging)),
+        "kernel_name": _native.kv_link_kernel_name(args),
     }
 
 
@@ -659,7 +660,7 @@ class PreparedKVLink:
     def launch(self) -> dict[str, Any]:
         """Kernel and launch shape of the link."""
 
-        return _launch_record(self._launch_info)
+        return _launch_record(self._args, self._launch_info)
 
     @staticmethod
     def _raise_for(error: _native.NativeCallError) -> None:
@@ -843,9 +844,9 @@ def describe_link_launch(
     if delta_workspace is not None:
         args.delta_workspace = delta_workspace.data_ptr()
         args.delta_workspace_bytes = delta_workspace.numel() * delta_workspace.element_size()
-    info = _native.kv_link_describe(args)
+    record = _launch_record(args, _native.kv_link_describe(args))
     del keepalive
-    return _launch_record(info)
+    return record
 
 
 class PreparedKVScatter:

@@ -448,8 +448,8 @@ int ll_order_link_maps(const ll_order_maps_args *args, ll_stream_t stream);
 /*
  * The same with every entry [prefix, count) in exact slot order (entries of one
  * slot in no fixed order): one launch more, through scratch_maps (device int64
- * [4, capacity], not overlapping maps or out_maps) and, with a mask,
- * scratch_mask (device uint8 [capacity]).  num_slots is at most 1,048,576 (64
+ * [4, capacity]) and, with a mask, scratch_mask (device uint8 [capacity]), which
+ * overlap none of the other arrays and not each other.  num_slots is at most 1,048,576 (64
  * slots per bucket).
  */
 int ll_order_link_maps_exact(const ll_order_maps_args *args, int64_t *scratch_maps, uint8_t *scratch_mask,

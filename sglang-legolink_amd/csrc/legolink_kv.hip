@@ -2462,6 +2462,15 @@ static int order_link_maps(const ll_order_maps_args *a, int64_t *scratch_maps, u
     if ((scratch < in_begin + bytes && in_begin < scratch + bytes) ||
         (scratch < out_begin + bytes && out_begin < scratch + bytes))
       return fail(LL_ERR_INVALID_ARGUMENT, "the scratch maps overlap maps or out_maps");
+    // The scratch mask against every array of the call: masks are bytes, maps 64-bit entries.
+    const uintptr_t entries = static_cast<uintptr_t>(a->capacity), m = reinterpret_cast<uintptr_t>(scratch_mask);
+    const auto overlaps = [&](const void *array, uintptr_t size) {
+      const uintptr_t first = reinterpret_cast<uintptr_t>(array);
+      return m < first + size && first < m + entries;
+    };
+    if (a->mask != nullptr && (overlaps(a->mask, entries) || overlaps(a->out_mask, entries) || overlaps(a->maps, bytes) ||
+                               overlaps(a->out_maps, bytes) || overlaps(scratch_maps, bytes)))
+      return fail(LL_ERR_INVALID_ARGUMENT, "the scratch mask overlaps a mask or maps of the call");
   }
   // One slot per bucket is an exact order already.
   const bool refine = exact && shift > 0 && a->count > a->prefix;

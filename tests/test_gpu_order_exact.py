@@ -146,3 +146,22 @@ def test_exact_order_refuses_what_it_cannot_take():
         args.num_slots = num_slots
         with pytest.raises(_native.NativeCallError, match=text):
             _native.order_link_maps_exact(args, scratch_maps, None, 0)
+
+
+def test_exact_order_refuses_a_scratch_mask_that_overlaps():
+    """Host checks only, as above: the scratch mask is read after the output mask is written."""
+
+    maps, out, scratch = (np.zeros(4 * 16, dtype=np.int64) for _ in range(3))
+    masks = np.zeros(16 * 3, dtype=np.uint8)
+    workspace = np.zeros(_native.ORDER_WORKSPACE_BYTES + 16, dtype=np.uint8)
+    args = _native.OrderMapsArgs()
+    args.maps, args.out_maps = maps.ctypes.data, out.ctypes.data
+    args.mask, args.out_mask = masks.ctypes.data, masks.ctypes.data + 16
+    args.capacity = args.count = 16
+    args.num_slots = 1 << 20
+    args.workspace = (workspace.ctypes.data + 15) // 16 * 16
+    args.workspace_bytes = _native.ORDER_WORKSPACE_BYTES
+    for mask in (args.mask, args.out_mask, args.mask + 15, args.out_mask - 1, args.out_mask + 15, maps.ctypes.data + 8,
+                 out.ctypes.data + 511, scratch.ctypes.data - 15):
+        with pytest.raises(_native.NativeCallError, match="scratch mask overlaps"):
+            _native.order_link_maps_exact(args, scratch.ctypes.data, mask, 0)

@@ -83,7 +83,8 @@ FORMS = {
     "half_rotary": _changed(rotary=lambda r: r // 2),
     "narrow_table": _changed(table=lambda t: t[:, :-2]),
     "flat_table": _changed(table=lambda t: t.flatten()),
-    "strided_table": _changed(table=lambda t: torch.cat([t, t], 1)[:, ::2].repeat(1, 2)[:, ::1]),
+    "strided_table": _changed(table=lambda t: t.repeat_interleave(2, 1)[:, ::2]),
+    "padded_table": _changed(table=lambda t: torch.cat([t, t], 1)[:, :t.shape[1]]),
     "int_table": _changed(table=lambda t: t.int()),
     "bf16_table": _changed(table=lambda t: t.bfloat16()),
     "parameter_layer": _changed(keys=_layer(0, lambda b: torch.nn.Parameter(b, requires_grad=False))),
@@ -107,6 +108,7 @@ def test_native_fill_agrees_with_the_python_checks(gpu_device, form, source):
         mask = torch.zeros(2 * n, device=gpu_device)
         inputs["mask"] = {"uint8": mask[:n].byte(), "bool": mask[:n].bool(), "float32": mask[:n],
                           "short": mask[: n - 1].byte(), "strided": mask.byte()[::2]}[kind]
+    assert form not in ("strided_table", "padded_table") or not inputs["table"].is_contiguous()
     filled, args, tables = _fill(inputs)
     expected = _python(inputs)
     # Taken only where the Python checks support the call; everything of this
@@ -229,6 +231,36 @@ def test_tensor_subclasses_take_the_python_path(gpu_device):
         destination_slots=inputs["dst"], local_positions=inputs["local"], global_positions=inputs["global"],
         cos_sin_cache=inputs["table"], prefix_token_count=0, rotary_dim=64, is_neox_style=True)
     assert torch.equal(inputs["values"][0][20:40], before[:20])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,step", [(3, 1), (3, 2), (1, 1)])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_native_write_back_fill_equals_the_python_one(gpu_device, monkeypatch, layers, step, index):
+    """Every field of the block, for dense and layer-strided rows."""
+
+    inputs = _inputs(gpu_device, layers=layers, vdim=32)
+    keys = torch.randn(6, 5, 2, 64, device=gpu_device).to(torch.bfloat16)[::step][:layers]
+    values = torch.randn(3, 5, 2, 32, device=gpu_device).to(torch.bfloat16)[:layers]
+    slots = torch.tensor([3, 49, 0, 7, 20], device=gpu_device, dtype=index)
+    args = _native.ScatterArgs()
+    tables = (ctypes.c_void_p * (2 * layers))()
+    assert _link_arguments.fill_scatter(ctypes.addressof(args), ctypes.addressof(tables), inputs["keys"],
+                                        inputs["values"], slots, keys, values)
+    prepared = []
+    for module in (_link_arguments, None):
+        monkeypatch.setattr(kv_link, "_link_arguments", module)
+        prepared.append(kv_link.PreparedKVScatter(key_buffers=inputs["keys"], value_buffers=inputs["values"],
+                                                  destination_slots=slots, repaired_keys=keys,
+                                                  repaired_values=values))
+    want = prepared[1]._args
+    args.struct_size, args.waves_per_block = want.struct_size, want.waves_per_block
+    for got in (args, prepared[0]._args):
+        for name, _ in _native.ScatterArgs._fields_:
+            field, expect = getattr(got, name), getattr(want, name)
+            if name in ("key_layers", "value_layers"):
+                field, expect = (list((ctypes.c_void_p * layers).from_address(a)) for a in (field, expect))
+            assert field == expect, name
 
 
 @pytest.mark.gpu

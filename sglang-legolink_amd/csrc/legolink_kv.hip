@@ -1180,9 +1180,12 @@ __global__ void __launch_bounds__(256) order_scatter_kernel(const OrderParams p)
 // The same three phases in one workgroup with its counters in LDS, for small
 // maps: one launch instead of three, and no phase waits for a kernel boundary.
 // Its time grows with the entries (one compute unit scatters them: 5.0 us for
-// 256, 6.8 for 1,024, 9.7 for 2,048, 15.9 for 4,096) where three launches take
-// 11.3 us; the line lies where one launch is still the faster one, and the host
-// saves two launches besides (a 2,048-token link as a whole 113 -> 108 us).
+// 256, 6.7 for 1,024, 9.7 for 2,048, 15.9 for 4,096) where three launches take
+// 11.3 us (2,049 entries, both replayed back to back from a graph); in the trace
+// of a link of 2,024 entries, between its other kernels, 11.2 against 3.1 + 6.2
+// + 4.4 and two gaps.  The line lies where one launch is still the faster one,
+// and the host saves two launches besides (a 2,048-token link as a whole 113 ->
+// 108 us).
 constexpr int kOrderSmallEntries = 2048;
 
 __global__ void __launch_bounds__(kOrderThreads) order_small_kernel(const OrderParams p) {

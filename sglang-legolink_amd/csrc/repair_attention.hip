@@ -166,8 +166,8 @@ __host__ __device__ constexpr int partial_floats() { return kQueries * D / 2 + 2
 // them: those with chunks below 512 keys, and those whose chunks split a tile
 // that the plan made without the head dim keeps whole (at head dim 256, whose
 // windows take two workgroups each).  The few partials of so small a plan cost
-// little (three spans over 2,048 keys 17.3 -> 17.9 us, 16.3 us
-// since the combine takes them in groups).
+// little (three spans over 2,048 keys 17.3 -> 17.9 us, 15.9 us since the combine
+// takes them in groups).
 template <int D>
 __device__ inline float *partial_block(const AttnParams &p, int partial, int h, bool wide) {
   return p.ws + (static_cast<long long>(partial) * p.hq + (wide ? 2 * h : h)) * partial_floats<D>();
@@ -354,7 +354,8 @@ __global__ void __launch_bounds__(m32_threads<D>()) repair_attention_m32_kernel(
   // trip away instead of three in a row.  With the slots and queries requested
   // together below, the time before the first tile is that of its ~850
   // instructions, no longer of a chain of loads: 15 spans over 32k keys (28/4
-  // heads) 74.5 -> 72.5 us, 168 spans of 24 requests 153.9 -> 153.2 us.
+  // heads) 74.1 -> 72.1 us, 168 spans of 24 requests 154.0 -> 152.6 us; many
+  // long items (c5's 511 spans, 3,470 us) gain nothing.
   static_assert(kItemInts > kWave && kItemInts <= 2 * kWave, "two fields per lane");
   // The kernel arguments in one group of scalar loads, ahead of their uses.
   asm volatile("" ::"s"(p.items), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.slots), "s"(p.positions), "s"(p.num_queries),
@@ -1011,7 +1012,7 @@ __global__ void __launch_bounds__(256 * kGroups) repair_combine_kernel(const Att
 }
 
 // Modelled run time of a plan in units of one 64-token key tile of a work
-// item (about 2.4 us for Qwen's 28/4 heads on MI355X).  `groups` calls its
+// item (2.3 us for Qwen's 28/4 heads on MI355X with every compute unit busy).  `groups` calls its
 // argument with (key tokens, partial results) of every group of query tiles.
 constexpr int kComputeUnits = 256;          // MI355X
 constexpr double kItemOverheadTiles = 3.0;  // slots, queries, write-out
@@ -1450,7 +1451,7 @@ int compute_plan(const ll_repair_row *rows, int64_t num_rows, int64_t num_q_head
     // 64 items, one round of 4 KV heads on 256 CUs, where 2,048 make 65).
     // Lengths below 512 where 512-key chunks leave compute units idle: three
     // 8-row spans over 2,048 keys (28/4 heads) take 24.2 us in 16 workgroups of
-    // 512 keys and 16.2 us in 52 of 128; where 512-key chunks fill the device,
+    // 512 keys and 15.9 us in 52 of 128; where 512-key chunks fill the device,
     // shorter ones only add rounds (15 spans over 32k keys: 108 us at 512, 122
     // at 384, 234 at 128).
     int64_t items_512 = 0;
